@@ -201,17 +201,60 @@ def _front(lanes, frames, seed):
 
 
 _tuned = set()    # shapes tuned in this process (the library's table is process-wide)
-_net = []         # the trained network, shared by the states of this process
+_net = []         # the network, shared by the states of this process
 
 
 def _network():
-    """A network trained as the benchmark trains it, on fewer pairs."""
-    if not _net:
-        pairs = Lr.generate_pairs(1024, 9, seed=101, snr=(4.0, 20.0), min_conf=0.0)
-        init = H.Initializer(seed=1)
-        Lr.train(init, pairs, epochs=10, batch=4096, lr=2e-3)
-        _net.append(init)
-    return _net[0]
+    """A network for the library, trained elsewhere (by torch, in 32 bits) on pairs of the plain pipeline with
+    the training recipe's loss, output map and schedule."""
+    if _net:
+        return _net[0]
+    pairs = Lr.generate_pairs(1024, 9, seed=101, snr=(4.0, 20.0), min_conf=0.0,
+                              gen_overrides={"empty_fraction": 0.05})
+    n = pairs.n
+    x = _view(pairs.x.data_ptr(), (n, H.MLP_IN), "<i2", pairs).view(torch.bfloat16).float()
+    t = _view(pairs.t.data_ptr(), (n, H.MLP_OUT), "<f4", pairs).clone()
+    v = _view(pairs.v.data_ptr(), (n,), "|u1", pairs).float()
+    t[v == 0, :11] = 0.0
+    tv = t[v > 0][:, :6]
+    offset, scale = tv.mean(0), tv.std(0).clamp(min=1e-3)
+    w = torch.tensor(Lr.LL_WEIGHTS, device="cuda") * scale ** 2 / Lr.LL_FRAMES
+    g = torch.Generator().manual_seed(1)
+    params = []
+    for n_out, n_in in ((256, 128), (256, 256), (12, 256)):
+        params.append(((2.0 * torch.rand(n_out, n_in, generator=g) - 1.0) * (6.0 / n_in) ** 0.5).cuda())
+        params.append(torch.zeros(n_out, device="cuda"))
+    for p in params:
+        p.requires_grad_()
+    opt = torch.optim.Adam(params, lr=2e-3)
+    batch, epochs = 4096, 10
+    steps = epochs * (n // batch)
+    for k in range(steps):
+        for group in opt.param_groups:
+            group["lr"] = 1e-4 + 1.9e-3 * 0.5 * (1.0 + float(np.cos(np.pi * k / steps)))
+        at = (k % (n // batch)) * batch
+        y = _forward(params, x[at:at + batch])
+        opt.zero_grad()
+        _loss(y, t[at:at + batch], v[at:at + batch], offset, scale, torch.cat([w, torch.ones(2, device="cuda")])).backward()
+        opt.step()
+    init = H.Initializer(seed=1)
+    init.set_params(torch.cat([p.detach().reshape(-1) for p in params]).cpu().numpy())
+    init.set_output_map(offset.tolist(), scale.tolist(), w.tolist() + [1.0, 1.0])
+    _net.append(init)
+    return init
+
+
+def _forward(params, x):
+    h = torch.relu(x @ params[0].t() + params[1])
+    h = torch.relu(h @ params[2].t() + params[3])
+    return h @ params[4].t() + params[5]
+
+
+def _loss(y, t, valid, offset, scale, w):
+    sq = (w[:6] * (y[:, :6] - (t[:, :6] - offset) / scale) ** 2).sum(1)
+    ce = -w[6] * (t[:, 6:11] * torch.log_softmax(y[:, 6:11], 1)).sum(1)
+    gate = w[7] * torch.nn.functional.binary_cross_entropy_with_logits(y[:, 11], t[:, 11], reduction="none")
+    return ((sq + ce) * valid + gate).mean()
 
 
 def _prepare_pool(case, seed):
@@ -555,15 +598,8 @@ def exact(case, seed):
         n = int(np.prod(shape))
         parts.append(p[at:at + n].view(shape).clone().requires_grad_())
         at += n
-    h = torch.relu(x @ parts[0].t() + parts[1])
-    h = torch.relu(h @ parts[2].t() + parts[3])
-    y = h @ parts[4].t() + parts[5]
     w = torch.tensor(NET_WEIGHTS, dtype=torch.float64, device=dev)
-    off, sc = offset.to(dev).double(), scale.to(dev).double()
-    sq = (w[:6] * (y[:, :6] - (t[:, :6] - off) / sc) ** 2).sum(1)
-    ce = -w[6] * (t[:, 6:11] * torch.log_softmax(y[:, 6:11], 1)).sum(1)
-    gate = w[7] * torch.nn.functional.binary_cross_entropy_with_logits(y[:, 11], t[:, 11], reduction="none")
-    loss = ((sq + ce) * v + gate).mean()
+    loss = _loss(_forward(parts, x), t, v, offset.to(dev).double(), scale.to(dev).double(), w)
     grads = torch.autograd.grad(loss, parts)
     one = loss.detach().view(1)
     return {"grads": torch.cat([g.reshape(-1) for g in grads]), "loss": one, "step_loss": one}
