@@ -201,17 +201,38 @@ struct HistView {
     __device__ uint32_t Cnt(int b) const { return (b < NB) ? (uint32_t)h->bin_count[b][z] : 0u; }
 };
 
-__device__ uint32_t InRange(const HistView& h, int* lastNonzero = nullptr)
+// Bins read at once by the set-up passes over a ZMW's counts: the loads of a batch are
+// all in flight together (a loop that tests each count before it loads the next waits for
+// memory at every bin: 90 of the 1070 us that one wave's estimate took).
+constexpr int kSetupBatch = 20;
+static_assert(NB % kSetupBatch == 0, "whole set-up batches");
+
+// Total of the in-range counts (16-bit, as UHistogramSimd adds them), the last nonempty bin
+// and the counts' sum as the EM's float accumulation gives it.
+__device__ uint32_t InRange(const HistView& h, int* lastNonzero, float* floatSum)
 {
     uint32_t s = 0;
     int last = -1;
-    for (int i = 0; i < NB; ++i) {
-        const uint32_t c = h.Cnt(i);
-        s = (s + c) & 0xffffu;
-        last = c ? i : last;
+#pragma unroll 1
+    for (int b = 0; b < NB; b += kSetupBatch) {
+        uint32_t c[kSetupBatch];
+#pragma unroll
+        for (int j = 0; j < kSetupBatch; ++j) c[j] = h.Cnt(b + j);
+#pragma unroll
+        for (int j = 0; j < kSetupBatch; ++j) {
+            s += c[j];
+            last = c[j] ? b + j : last;
+        }
     }
-    if (lastNonzero) *lastNonzero = last;
-    return s;
+    *lastNonzero = last;
+    // Every partial sum below 2^24 is exact in float, so the order does not matter there.
+    float f = (float)s;
+    if (s >= (1u << 24)) {
+        f = 0.0f;
+        for (int b = 0; b < NB; ++b) f += (float)h.Cnt(b);
+    }
+    *floatSum = f;
+    return s & 0xffffu;
 }
 
 // UHistogramSimd::CumulativeCount (UHistogramSimd.cpp:199-238)
@@ -222,13 +243,20 @@ __device__ float CumulativeCount(const HistView& h, uint32_t lowOut, uint32_t in
     const bool mHigh = x >= h.Start(NB);
     const bool mIn = !(mNan || mLow || mHigh);
     int xbin = hw_floor_i32((x - h.Start(0)) / h.bs);
-    if (!mIn) xbin = 0;
+    if (!mIn || xbin < 0) xbin = 0;   // (x inside NaN bounds: the quotient is NaN, and so is the result)
     const float xrem = x - h.Start(xbin);
     const float xbinCount = (float)h.Cnt(xbin);
     float cc = (float)lowOut;
     uint32_t below = 0;
-    for (int i = 0; i < xbin; ++i) below = (below + h.Cnt(i)) & 0xffffu;
-    cc += (float)below;
+#pragma unroll 1
+    for (int b = 0; b < NB && __any(b < xbin); b += kSetupBatch) {
+        uint32_t c[kSetupBatch];
+#pragma unroll
+        for (int j = 0; j < kSetupBatch; ++j) c[j] = h.Cnt(b + j);
+#pragma unroll
+        for (int j = 0; j < kSetupBatch; ++j) below += (b + j < xbin) ? c[j] : 0u;
+    }
+    cc += (float)(below & 0xffffu);
     cc += xbinCount * xrem / h.bs;
     if (mLow) cc = (float)lowOut;
     if (mHigh) cc = (float)((lowOut + inRange) & 0xffffu);
@@ -242,12 +270,28 @@ __device__ float Fractile(const HistView& h, uint32_t lowOut, uint32_t total, fl
     const float nfz = frac * (float)total;
     uint32_t n = lowOut;
     if (n > 0 && (float)n >= nfz) return hw_u2f(0xff800000u);
+    // The first bin at which the running count (mod 2^16) is positive and reaches nfz.
     int i = 0;
-    while ((n == 0 || (float)n < nfz) && i < NB) n = (n + h.Cnt(i++)) & 0xffffu;
+    uint32_t niz = 0;
+    bool go = n == 0 || (float)n < nfz;
+#pragma unroll 1
+    for (int b = 0; b < NB && __any(go); b += kSetupBatch) {
+        uint32_t c[kSetupBatch];
+#pragma unroll
+        for (int j = 0; j < kSetupBatch; ++j) c[j] = h.Cnt(b + j);
+#pragma unroll
+        for (int j = 0; j < kSetupBatch; ++j) {
+            if (go) {
+                n = (n + c[j]) & 0xffffu;
+                niz = c[j];
+                ++i;
+                go = n == 0 || (float)n < nfz;
+            }
+        }
+    }
     if ((float)n < nfz) return hw_u2f(0x7f800000u);
-    i -= 1;
+    i -= 1;   // -1 (no bin taken) only for a NaN fraction, whose result is NaN
     const float x0 = h.Start(i);
-    const uint32_t niz = h.Cnt(i);
     const int m = (int)n - (int)niz;
     return x0 + h.bs * (nfz - (float)m) / (float)(niz + 1);
 }
@@ -280,8 +324,16 @@ struct EmExtra {
 constexpr float kExpZeroBelow = -105.0f;
 // Boundaries per exact restart of the density recurrence of the E-step.
 constexpr int kRecurBlock = 10;
-// Bins between a count's load and its use in the E-step.
-constexpr int kCntAhead = 2;
+// hw_expf without its clamp and its NaN case, for finite t in [-8e6, 200] (and any t whose
+// result is not used): the same steps, so the same bits.  Below -200 the clamp only keeps k in
+// range: t log2(e) is within 0.7 of its rounded value there, so |r| < 0.9, exp(r)'s polynomial is
+// positive and 2^k times it is +0, as with the clamp.
+__device__ __forceinline__ float ExpBounded(float t)
+{
+    const float kf = hw_rintf(t * 1.44269502162933349609375f);
+    const float r = hw_fmaf(-kf, 1.428606765330187045e-06f, hw_fmaf(-kf, 0.693145751953125f, t));
+    return hw_ldexpf(hw_exp_poly(r), (int)kf);
+}
 
 template <int MODE>
 __global__ __launch_bounds__(64, 3) void DmeEstimateKernel(const hwpa_lane_hist* __restrict__ hists,
@@ -320,7 +372,8 @@ __global__ __launch_bounds__(64, 3) void DmeEstimateKernel(const hwpa_lane_hist*
     HistView h{&lh, z, lh.low_bound[z], lh.bin_size[z]};
     const uint32_t lowOut = lh.outlier_low[z], highOut = lh.outlier_high[z];
     int lastNz;
-    const uint32_t inRange = InRange(h, &lastNz);
+    float njSum;
+    const uint32_t inRange = InRange(h, &lastNz, &njSum);
     const uint32_t numFrames = (inRange + ((lowOut + highOut) & 0xffffu)) & 0xffffu;
 
     const float rpa[NA] = {d.relAmp[0], d.relAmp[1], d.relAmp[2], d.relAmp[3]};
@@ -416,8 +469,6 @@ __global__ __launch_bounds__(64, 3) void DmeEstimateKernel(const hwpa_lane_hist*
     int status = (numFrames < 160u) ? HWPA_ZS_INSUF_DATA : HWPA_ZS_OK;
     bool converged = false;
     float mlLogLike = hw_u2f(0xff800000u);
-    float njSum = 0.0f;
-    for (int b = 0; b < NB; ++b) njSum += (float)h.Cnt(b);
     const float halfBin = 0.5f * h.bs;
     int iterLimit = d.iterLimit;
     if (MODE == EM_LEARNED) {
@@ -494,80 +545,127 @@ __global__ __launch_bounds__(64, 3) void DmeEstimateKernel(const hwpa_lane_hist*
         // restart is below FLT_MIN while rising, or whose ratio exceeds e^80, takes exp
         // at every boundary of the block (a density coming out of underflow cannot be
         // continued from +0).
-        float dd[5], rr[5], qq[5];
+        float dd[5], rr[5], qq[5], nbs[5];
 #pragma unroll
-        for (int k = 0; k < 5; ++k) qq[k] = hw_expf((2.0f * nhv[k]) * (h.bs * h.bs));
-        uint32_t exMask = 0;
-        bool anyEx = false;   // some ZMW of the wave takes exp at every boundary of this block
+        for (int k = 0; k < 5; ++k) {
+            qq[k] = hw_expf((2.0f * nhv[k]) * (h.bs * h.bs));
+            nbs[k] = nhv[k] * h.bs;
+        }
         auto tAt = [&](float x, int i) {
             const float y = x - mu[i];
             return hw_fmaf(y * y, nhv[i], pref[i]);
         };
-        float nbs[5];
+        // Whether every exponent of this iteration's restarts lies in [-8e6, 200] for all ZMWs
+        // of the wave: then ExpBounded serves them (not the case only for degenerate models or
+        // bounds: NaN, infinite, zero or negative variances).
+        bool bounded = true;
 #pragma unroll
-        for (int k = 0; k < 5; ++k) nbs[k] = nhv[k] * h.bs;
-        auto restart = [&](int c) {
+        for (int i = 0; i < 5; ++i) {
+            const float far = __builtin_fmaxf(hw_fabsf(h.lb - mu[i]), hw_fabsf(h.Start(NB) - mu[i]));
+            bounded = bounded && nhv[i] <= 0.0f && (far * far) * nhv[i] >= -4e6f && pref[i] <= 80.0f && pref[i] >= -1e6f;
+        }
+        bounded = __all(bounded);
+        uint32_t exMask = 0;   // this ZMW's components that take exp at every boundary of the block
+        uint32_t exAny = 0;    // the same for any ZMW of the wave
+        bool zeroBl = false;   // the baseline density is +0 through the block for the whole wave
+        auto restart = [&](int c, auto expOf) {
             const float x0 = h.Start(c);
-            exMask = 0;
+            float dl[5];
 #pragma unroll
             for (int i = 0; i < 5; ++i) {
                 const float y0 = x0 - mu[i];
                 const float t0 = hw_fmaf(y0 * y0, nhv[i], pref[i]);
                 // t(x0 + bs) - t(x0) on the ideal grid (no cancellation of rounded t)
-                const float dl = nbs[i] * hw_fmaf(2.0f, y0, h.bs);
+                dl[i] = nbs[i] * hw_fmaf(2.0f, y0, h.bs);
                 // exp(t) is +0 below the threshold: waves skip the exp when all ZMWs are, and
                 // then the ratio's too.  The density stays +0 through the block (+0 times any
                 // finite ratio >= 0); a rising one (dl > 0) takes exp at every boundary below.
-                if (__all(t0 < kExpZeroBelow)) {
+                const bool zero = __all(t0 < kExpZeroBelow);
+                if (i == 0) zeroBl = zero;
+                if (zero) {
                     dd[i] = 0.0f;
                     rr[i] = 0.0f;
                 } else {
-                    dd[i] = hw_expf(t0);
-                    rr[i] = hw_expf(dl);
+                    dd[i] = expOf(t0);
+                    rr[i] = expOf(dl[i]);
                 }
-                const bool rec = (dd[i] >= FLT_MIN || dl <= 0.0f) && dl <= 80.0f;
-                exMask |= (rec ? 0u : 1u) << i;
             }
-            anyEx = __any(exMask != 0u);
-        };
-        auto advance = [&](int c) {
+            // No ZMW leaves the recurrence when every density is at least FLT_MIN or falling
+            // (max(dd, -dl) >= FLT_MIN) and no ratio is above e^80; the comparisons are false
+            // for NaN, which takes the exact test.
+            float lo = __builtin_fmaxf(dd[0], -dl[0]), hi = dl[0];
 #pragma unroll
-            for (int i = 0; i < 5; ++i) {
+            for (int i = 1; i < 5; ++i) {
+                lo = __builtin_fminf(lo, __builtin_fmaxf(dd[i], -dl[i]));
+                hi = __builtin_fmaxf(hi, dl[i]);
+            }
+            exMask = 0;
+            exAny = 0;
+            if (!bounded || !__all(lo >= FLT_MIN && hi <= 80.0f)) {
+                // A component that starts the block below the zero threshold and is still
+                // below it, and still left of its mean, at the block's end has +0 for every
+                // exp in between (t rises up to the mean; the threshold leaves a margin of 1
+                // for its rounding): the recurrence from +0 gives the same, with a ratio of 0.
+                const float x1 = h.Start(c + kRecurBlock);
+#pragma unroll
+                for (int i = 0; i < 5; ++i) {
+                    const bool rec = (dd[i] >= FLT_MIN || dl[i] <= 0.0f) && dl[i] <= 80.0f;
+                    const bool flat = tAt(x0, i) < kExpZeroBelow && tAt(x1, i) < kExpZeroBelow && x1 <= mu[i];
+                    if (!rec && flat) rr[i] = 0.0f;
+                    const bool ex = !rec && !flat;
+                    exMask |= (ex ? 1u : 0u) << i;
+                    exAny |= (__any(ex) ? 1u : 0u) << i;
+                }
+                exAny = __builtin_amdgcn_readfirstlane(exAny);
+                zeroBl = zeroBl && (exAny & 1u) == 0u;
+            }
+        };
+        // One boundary c with densities dd and the count n of the bin before it: that bin's
+        // probability, its term of the log-likelihood and f = n / binp, then the sums of
+        // boundary c - 1 with weight F = f_{c-2} + f_{c-1}.  Where the wave's counts are all
+        // zero the terms are exact zeros (every density is finite) and may be left out.
+        float bpPrev = 0.0f, fPrev = 0.0f, dPrev[5] = {0.f, 0.f, 0.f, 0.f, 0.f};
+        auto binProb = [&](int c, bool bl) {
+            const float a0 = bl ? dd[0] + dd[1] : dd[1];
+            const float bp = a0 + (dd[2] + (dd[3] + dd[4]));   // Sum5Tree
+            // binp >= binProbMin >= FLT_MIN and finite: the log needs no special cases
+            const float binp = hw_max_pos(halfBin * (bpPrev + bp), binProbMin);
+            probSum = c == 0 ? 0.0f : probSum + binp;   // (there is no bin before boundary 0)
+            bpPrev = bp;
+            return binp;
+        };
+        auto weigh = [&](float binp, uint32_t n) {
+            const float nj = (float)n;
+            float lg, rcp;
+            hw_log_rcp_tab(binp, sRc, sLc, &lg, &rcp);
+            wps = hw_fmaf(nj, lg, wps);
+            return nj * rcp;
+        };
+        auto gather = [&](float x, float F, bool bl) {
+            const float G = x * F;
+#pragma unroll
+            for (int m = bl ? 0 : 1; m < 5; ++m) {
+                ci[m] = hw_fmaf(dPrev[m], F, ci[m]);
+                mom1[m] = hw_fmaf(dPrev[m], G, mom1[m]);
+            }
+            if (bl) {
+                const float dev = x - piv;
+                const float w = dPrev[0] * F;
+                q1 = hw_fmaf(w, dev, q1);
+                q2 = hw_fmaf(w * dev, dev, q2);
+            }
+        };
+        auto keep = [&]() {
+#pragma unroll
+            for (int m = 0; m < 5; ++m) dPrev[m] = dd[m];
+        };
+        auto advance = [&](bool bl) {
+#pragma unroll
+            for (int i = bl ? 0 : 1; i < 5; ++i) {
                 dd[i] = dd[i] * rr[i];
                 rr[i] = rr[i] * qq[i];
             }
-            if (anyEx) {
-                const float x = h.Start(c);
-#pragma unroll
-                for (int i = 0; i < 5; ++i)
-                    if ((exMask >> i) & 1u) dd[i] = hw_expf(tAt(x, i));
-            }
         };
-        // Sums of boundary c with weight F = f_{c-1} + f_c; skipped when F is 0 for the
-        // whole wave (every density is finite, so the terms are exact zeros).
-        auto gather = [&](const float* dc, float x, float F) {
-            if (__all(F == 0.0f)) return;
-            const float G = x * F;
-#pragma unroll
-            for (int m = 0; m < 5; ++m) {
-                ci[m] = hw_fmaf(dc[m], F, ci[m]);
-                mom1[m] = hw_fmaf(dc[m], G, mom1[m]);
-            }
-            const float dev = x - piv;
-            const float w = dc[0] * F;
-            q1 = hw_fmaf(w, dev, q1);
-            q2 = hw_fmaf(w * dev, dev, q2);
-        };
-        restart(0);
-        float bpPrev = Sum5Tree(dd), dPrev[5];
-#pragma unroll
-        for (int m = 0; m < 5; ++m) dPrev[m] = dd[m];
-        float fPrev = 0.0f;
-        // Bin counts kCntAhead bins ahead, so their loads are in flight over that many bins.
-        uint32_t cq[kCntAhead];
-#pragma unroll
-        for (int j = 0; j < kCntAhead; ++j) cq[j] = h.Cnt(j);
-        static_assert(NB % kRecurBlock == 0, "whole blocks of boundaries");
         // The tail of the histogram is left out once, for every ZMW of the wave, the bins
         // ahead are empty, the boundary lies beyond every mode's mean (so each density
         // only falls from here on) and bs times the density sum is below 2^-27 of
@@ -578,45 +676,90 @@ __global__ __launch_bounds__(64, 3) void DmeEstimateKernel(const hwpa_lane_hist*
         float maxMu = mu[0];
 #pragma unroll
         for (int k = 1; k < 5; ++k) maxMu = hw_maxf(maxMu, mu[k]);
-        int bEnd = NB;
-        for (int b0 = 0; b0 < NB; b0 += kRecurBlock) {
+        // Counts of a block's bins b0 - 1 .. b0 + 8, each read again for the next block as
+        // soon as it has been used, so its load is in flight over a whole block.
+        uint32_t cn[kRecurBlock];
+#pragma unroll
+        for (int j = 0; j < kRecurBlock; ++j) cn[j] = (j == 0) ? 0u : h.Cnt(j - 1);
+        int cLast = NB;   // the last boundary taken
+#pragma unroll 1
+        for (int b0 = 0; b0 <= NB; b0 += kRecurBlock) {
             if (b0 > 0) {
                 const float tol = hw_ldexpf(probSum, -27);
-                const bool tail = lastNz < b0 && h.Start(b0) > maxMu && h.bs * bpPrev < tol && binProbMin < tol;
+                const bool tail = lastNz < b0 - 1 && h.Start(b0 - 1) > maxMu && h.bs * bpPrev < tol && binProbMin < tol;
                 if (__all(tail)) {
-                    bEnd = b0;
+                    cLast = b0 - 1;
                     break;
                 }
             }
-#pragma unroll
-            for (int j = 0; j < kRecurBlock; ++j) {
-                const int b = b0 + j;
-                const uint32_t cnt = cq[0];
-#pragma unroll
-                for (int q = 0; q + 1 < kCntAhead; ++q) cq[q] = cq[q + 1];
-                cq[kCntAhead - 1] = h.Cnt(b + kCntAhead);
-                if (j == kRecurBlock - 1) restart(b + 1);
-                else advance(b + 1);
-                const float bpNext = Sum5Tree(dd);
-                // binp >= binProbMin >= FLT_MIN and finite: the log needs no special cases
-                const float binp = hw_max_pos(halfBin * (bpPrev + bpNext), binProbMin);
-                probSum += binp;
-                float f = 0.0f;   // n_b / binp_b, +0 for an empty bin
-                if (!__all(cnt == 0u)) {
-                    const float nj = (float)cnt;
-                    float lg, rcp;
-                    hw_log_rcp_tab(binp, sRc, sLc, &lg, &rcp);
-                    wps = hw_fmaf(nj, lg, wps);
-                    f = nj * rcp;
-                }
-                gather(dPrev, h.Start(b), fPrev + f);
-                bpPrev = bpNext;
-#pragma unroll
-                for (int m = 0; m < 5; ++m) dPrev[m] = dd[m];
+            if (bounded) restart(b0, [](float t) { return ExpBounded(t); });
+            else restart(b0, [](float t) { return hw_expf(t); });
+            if (b0 == NB) {   // the last boundary: bin NB - 1
+                const float f = weigh(binProb(NB, true), h.Cnt(NB - 1));
+                gather(h.Start(NB - 1), fPrev + f, true);
                 fPrev = f;
+                keep();
+                break;
+            }
+            uint32_t none = 0;   // bins empty for the whole wave
+#pragma unroll
+            for (int j = 0; j < kRecurBlock; ++j) none |= (__all(cn[j] == 0u) ? 1u : 0u) << j;
+            none = __builtin_amdgcn_readfirstlane(none);
+            // Row of the next block's first bin (the last block's own is read when it is needed).
+            const uint16_t* ahead = &h.h->bin_count[min(b0 + kRecurBlock - 1, NB - kRecurBlock)][z];
+            if (exAny != 0u || __popc(none) > 1) {
+                // Some component takes exp at every boundary, or bins are empty for the whole
+                // wave: both are left to wave-uniform branches.
+                bool noF = __all(fPrev == 0.0f);
+#pragma unroll
+                for (int j = 0; j < kRecurBlock; ++j) {
+                    if (j > 0) {
+                        advance(true);
+                        if (exAny != 0u) {
+                            const float x = h.Start(b0 + j);
+#pragma unroll
+                            for (int i = 0; i < 5; ++i) {
+                                if ((exAny >> i) & 1u) {
+                                    const float v = hw_expf(tAt(x, i));
+                                    dd[i] = ((exMask >> i) & 1u) ? v : dd[i];
+                                }
+                            }
+                        }
+                    }
+                    const float binp = binProb(b0 + j, true);
+                    const bool empty = (none >> j) & 1u;
+                    if (!(empty && noF)) {
+                        const float f = empty ? 0.0f : weigh(binp, cn[j]);
+                        gather(h.Start(b0 + j - 1), fPrev + f, true);
+                        fPrev = f;
+                    }
+                    noF = empty;
+                    keep();
+                    cn[j] = ahead[j * LS];
+                }
+            } else if (zeroBl) {
+#pragma unroll
+                for (int j = 0; j < kRecurBlock; ++j) {
+                    if (j > 0) advance(false);
+                    const float f = weigh(binProb(b0 + j, false), cn[j]);
+                    gather(h.Start(b0 + j - 1), fPrev + f, j == 0);
+                    fPrev = f;
+                    keep();
+                    cn[j] = ahead[j * LS];
+                }
+            } else {
+#pragma unroll
+                for (int j = 0; j < kRecurBlock; ++j) {
+                    if (j > 0) advance(true);
+                    const float f = weigh(binProb(b0 + j, true), cn[j]);
+                    gather(h.Start(b0 + j - 1), fPrev + f, true);
+                    fPrev = f;
+                    keep();
+                    cn[j] = ahead[j * LS];
+                }
             }
         }
-        gather(dPrev, h.Start(bEnd), fPrev);
+        gather(h.Start(cLast), fPrev, true);
         const float q0 = ci[0];
 #pragma unroll
         for (int m = 0; m < 5; ++m) {

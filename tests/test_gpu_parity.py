@@ -302,6 +302,38 @@ def test_dme_estimate_recurrence_edge_paths_bit_exact(H, O, T, gpu):
     _eq_struct(H.to_numpy(d_models, T.LANE_MODEL, (L,)), o_models, "models")
 
 
+@pytest.mark.parametrize("shape", ["full_counters", "few_bins", "far_bounds"])
+def test_dme_estimate_block_paths_bit_exact(H, O, T, gpu, shape):
+    """The E-step's block forms against the oracle: counters whose sum passes 2^24 (every bin
+    full), bins empty for a whole lane between occupied ones (branch per bin), and bins so wide
+    that the restarts' exponents leave the range of the unclamped exp."""
+    L, F = 4, 512
+    cfg, h, s, m = _em_case(H, O, T, L, F, 5)
+    h = h.copy()
+    if shape == "full_counters":
+        h["bin_count"][0] = 65535
+        h["bin_count"][1, 100:] = 65000
+        h["outlier_low"][0] = 3
+    elif shape == "few_bins":
+        keep = np.zeros(300, bool)
+        keep[[3, 17, 18, 19, 24, 25, 40, 41, 60, 95, 96, 97, 150, 299]] = True
+        h["bin_count"][0:3, ~keep] = 0
+        h["bin_count"][1, 120:] = 0
+        h["bin_count"][2, :20] = 0
+        h["bin_count"][0:3, 18] += 150
+    else:
+        h["bin_size"][0:2, 5::16] *= np.float32(3e3)
+        h["low_bound"][1, 7::16] = np.float32(-3e5)
+    mfi, efi = (512, 1024), (1024, 1536)
+    o_models, diag = O.dme_estimate(cfg, h, s, m, mfi, efi, want_diag=True, form="mirror")
+    d_models = _dev(H, m)
+    d_iters = H.dev_bytes(L * 4)
+    H.dme_estimate(cfg, _dev(H, h), _dev(H, s), d_models, mfi, efi, L, d_iters)
+    iters = H.to_numpy(d_iters, np.int32, (L,))
+    assert list(iters) == [diag[l].iterations_run for l in range(L)]
+    _eq_struct(H.to_numpy(d_models, T.LANE_MODEL, (L,)), o_models, "models")
+
+
 @pytest.fixture(params=[0, 1, 2, 3])
 def label_variant(request, H):
     """Every autotuner variant of the labeler (16 or 8 frames per batch, registers
