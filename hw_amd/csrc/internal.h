@@ -83,7 +83,7 @@ int32_t HistAddWrap(hwpa_lane_hist* hist, void* edge, const int16_t* traces, uin
                     const hwpa_lane_model* models, uint32_t lanes, hipStream_t s);
 
 // Kernel shape variants chosen per (lanes, frames) by the autotuner; every
-// variant computes the same bits.  Variant 0 is the default.
+// variant computes the same bits.  Variant 0 is the choice by size, for shapes not tuned.
 enum TuneKernel { kTuneHistogram = 0, kTuneBaseline = 1, kTuneLabel = 2, kTunePulse = 3, kTuneKernels = 4 };
 int32_t TuneVariants(int kernel);
 int32_t TuneGet(int kernel, uint32_t lanes, uint32_t frames);

@@ -291,12 +291,15 @@ int32_t PulserRun(PulserDev* p, const int16_t* labels, const int16_t* latent, co
 #define HWPA_PULSE_LAUNCH(U, PF, Q)                                                                               \
     hipLaunchKernelGGL((PulseKernel<U, PF, Q>), dim3(p->lanes), dim3(LS), 0, s, labels, latent, traces, (int)frames, \
                        first_frame, models, p->seg, pulses, counts, overflows, bl_stats, p->k)
-    // Variants: frames per batch x batches in the load ring x queued record writing.
+    // Variants: frames per batch x batches in the load ring x queued record writing.  0, the choice
+    // for shapes that were not tuned, is the queued 8 x 2 form: the fastest or within 2% of it at
+    // every shape measured, 16 to 16,384 lanes x 128 to 1024 frames (records written at the frame
+    // that ends them, 8 x 1, the earlier choice: 206 against 104 us at 64 lanes x 512 frames, 501
+    // against 302 at 4,096, 1680 against 1154 at 16,384).
     switch (TuneGet(kTunePulse, p->lanes, frames)) {
     case 1: HWPA_PULSE_LAUNCH(8, 2, false); break;
     case 2: HWPA_PULSE_LAUNCH(16, 2, false); break;
     case 3: HWPA_PULSE_LAUNCH(8, 1, true); break;
-    case 4: HWPA_PULSE_LAUNCH(8, 2, true); break;
     case 5: HWPA_PULSE_LAUNCH(4, 2, true); break;
     case 6: HWPA_PULSE_LAUNCH(4, 1, true); break;
     case 7: HWPA_PULSE_LAUNCH(4, 4, true); break;
@@ -305,7 +308,7 @@ int32_t PulserRun(PulserDev* p, const int16_t* labels, const int16_t* latent, co
     case 10: HWPA_PULSE_LAUNCH(4, 12, true); break;
     case 11: HWPA_PULSE_LAUNCH(8, 4, true); break;
     case 12: HWPA_PULSE_LAUNCH(2, 16, true); break;
-    default: HWPA_PULSE_LAUNCH(8, 1, false); break;
+    default: HWPA_PULSE_LAUNCH(8, 2, true); break;   // 0 and 4
     }
 #undef HWPA_PULSE_LAUNCH
     return CheckLaunch("PulseKernel");

@@ -143,15 +143,16 @@ int32_t hwpa_batch_autotune(hwpa_batch* b, int32_t repeats);
 /* ---- kernel-shape autotuner (no reference counterpart) -------------------
  * Tunable kernels run in variants that give the same bits with different
  * shapes: kernel 0 = histogram (variants 0-8: one wave per lane, 8, 16 or 32
- * frames per prefetched batch x 128, 160 or 192 bins kept in LDS; 9-15: 2, 4 or
+ * frames per prefetched batch x 128, 160 or 192 bins kept in LDS, but 0 is the form
+ * chosen by default; 9-15: 2, 4 or
  * 8 waves per lane sharing its LDS counters; 16-21: all 300 bins in LDS, 8 or 16
  * frames per batch x 4, 8 or 2 waves per lane), kernel 1 = baseline filter (1, 2 or 4 lanes per
  * workgroup, then the same with two groups of raw frames in flight), kernel 2 = Viterbi labeler (16 or 8 frames per prefetched
  * batch, then the same with registers held to 4 waves per SIMD), kernel 3 = pulse accumulator (frames
- * per batch x batches in the load ring x record queue: 8x1, 8x2, 16x2 writing records directly; 8x1,
- * 8x2, 4x2, 4x1, 4x4, 8x3, 4x8, 4x12, 8x4, 2x16 writing them through an LDS queue).
+ * per batch x batches in the load ring x record queue: the default, then 8x2, 16x2 writing records
+ * directly; 8x1, 8x2, 4x2, 4x1, 4x4, 8x3, 4x8, 4x12, 8x4, 2x16 writing them through an LDS queue).
  * The launchers look up the variant for their (lanes, frames);
- * unset shapes use variant 0.  hwpa_autotune times every variant on
+ * unset shapes use variant 0, the library's choice by the shape's size.  hwpa_autotune times every variant on
  * synthetic traces of the shape (`repeats` timed runs each, HIP events) and
  * keeps the fastest; ms (optional, ms_len entries) receives the mean times
  * of the variants of kernel 0, then 1, 2 and 3. */
