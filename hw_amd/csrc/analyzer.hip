@@ -750,6 +750,9 @@ int32_t hwpa_batch_create(uint32_t n_pools, const uint32_t* pool_ids, const uint
         }
         b->pools.push_back(a);
     }
+    uint64_t allLanes = 0;
+    for (auto* a : b->pools) allLanes += a->lanes;
+    for (auto* a : b->pools) LabelerShare(a->lab, allLanes);
     b->joins.assign(n_pools, nullptr);
     bool ok = hipStreamCreate(&b->master) == hipSuccess;
     ok = ok && hipEventCreateWithFlags(&b->fork, hipEventDisableTiming) == hipSuccess;

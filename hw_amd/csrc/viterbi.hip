@@ -4,7 +4,8 @@
 // traceAnalysis/SubframeScorer.h:143-318; ROI, traceAnalysis/RoiHost.h:75-248;
 // transition matrix, traceAnalysis/SubframeScorer.cpp:35-223).
 //
-// Mapping: one wave64 per lane, one thread per ZMW, sequential over frames.
+// Mapping: one wave64 per lane, one thread per ZMW (four in small pools, see LabelQuadKernel),
+// sequential over frames.
 // The ROI is computed first (forward hysteresis, then a backward pass) into a
 // 2-bit-per-frame LDS array; the recursion then runs over latent + chunk +
 // stitch frames.  The transition matrix has a fixed sparsity (each row: one
@@ -17,6 +18,7 @@
 
 #include "internal.h"
 
+#include <algorithm>
 #include <cmath>
 
 namespace hwpa {
@@ -39,9 +41,20 @@ struct LabelerDev {
     TransVals T;
     float roiUpper, roiLower;
     uint32_t lanes, maxFrames;
+    bool quad = false;       // the buffer holds LabelQuadKernel's words too
     LabLaneState* state = nullptr;
-    uint32_t* tb = nullptr;  // [lane][maxFrames + 16 + NS][LS]: predecessor words, then the anchor row
+    uint32_t* tb = nullptr;  // [lane][maxFrames + 16 + NS][LS]: predecessor words, then the anchor row;
+                             // or (quad) 64-bit words [lane][maxFrames + 16][LS]
 };
+
+// Pools of at most this many lanes are labeled by four threads per ZMW (LabelQuadKernel).  It
+// issues 1.5 times the instructions of LabelKernel, in waves 2.6 times shorter, so it wins until
+// its waves fill the chip's issue slots (512 frames, quad against one thread per ZMW): 16 lanes
+// 0.20 against 0.50 ms, 512 lanes 0.32 against 0.52, 1,024 lanes 0.55 against 0.54, 4,096 lanes
+// 1.9 against 1.2.  Pools that run side by side fill the chip together, so they count together
+// (six pools of 365 to 2,048 lanes in one graph: 7.1 ms a step, 7.3 with the two below 768 lanes
+// on four threads).
+constexpr uint32_t kQuadLanes = 768;
 
 // nhB = -1/(2 var_B), nhP = -1/(2 var_a): the reference's -0.5f * y * invVar * y
 // equals (y * (-0.5f * invVar)) * y bit for bit (scaling by -0.5 is exact here).
@@ -457,6 +470,467 @@ __global__ __launch_bounds__(64, MINW) void LabelKernel(const int16_t* __restric
     st.oldModel.confidence[z] = model.confidence[z];
 }
 
+// ---- four threads per ZMW -----------------------------------------------------
+// For pools that leave the chip partly idle: a quad of lanes carries one ZMW, thread a of it the
+// states of analog a (full_a, up_a, down_a; the baseline state is kept by all four), so a wave
+// holds 16 ZMWs and a frame costs it 168 instructions instead of 440.  Values cross the quad by DPP.  A frame's predecessor choices are one 64-bit word per
+// ZMW, 16 bits from each thread: the nibbles of full_a, up_a, down_a and the baseline, at the
+// state's own nibble index (4a, 4a + 1, 4a + 2; 3 for the baseline), each holding the
+// predecessor's index, so a traceback step is one shift of that word.
+// Every value is formed as LabelKernel forms it, so both give the same bits.
+
+template <int CTRL>
+__device__ __forceinline__ uint32_t QuadU(uint32_t v)
+{
+    return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, CTRL, 0xf, 0xf, true);
+}
+template <int CTRL>
+__device__ __forceinline__ float QuadF(float v) { return hw_u2f(QuadU<CTRL>(hw_f2u(v))); }
+constexpr int kQuadXor1 = 0xB1, kQuadXor2 = 0x4E;
+// Value of quad thread P.
+template <int P>
+__device__ __forceinline__ float QuadAt(float v) { return QuadF<P * 0x55>(v); }
+__device__ __forceinline__ float QuadAt(float v, int p)
+{
+    return p == 0 ? QuadAt<0>(v) : p == 1 ? QuadAt<1>(v) : p == 2 ? QuadAt<2>(v) : QuadAt<3>(v);
+}
+__device__ __forceinline__ uint32_t QuadAtU(uint32_t v, int p)
+{
+    return p == 0 ? QuadU<0x00>(v) : p == 1 ? QuadU<0x55>(v) : p == 2 ? QuadU<0xAA>(v) : QuadU<0xFF>(v);
+}
+__device__ __forceinline__ uint32_t QuadOr(uint32_t v)
+{
+    v |= QuadU<kQuadXor1>(v);
+    return v | QuadU<kQuadXor2>(v);
+}
+__device__ __forceinline__ uint32_t QuadMaxU(uint32_t v)
+{
+    v = max(v, QuadU<kQuadXor1>(v));
+    return max(v, QuadU<kQuadXor2>(v));
+}
+
+constexpr uint32_t kNibB = 3;   // nibble index of the baseline state
+// State number of a nibble index: full_a 1 + a, up_a 5 + a, down_a 9 + a, the baseline 0.
+__device__ __forceinline__ int NibState(uint32_t n)
+{
+    const int k = (int)(n & 3u);
+    return k == 3 ? 0 : 1 + (int)(n >> 2) + 4 * k;
+}
+__device__ __forceinline__ uint32_t StateNib(int s) { return s == 0 ? kNibB : 4u * (uint32_t)((s - 1) & 3) + (uint32_t)((s - 1) >> 2); }
+
+struct ScorerQ {   // ScorerZ's values for the baseline and one analog
+    float bgMean, nhB, bgFixed, x0;
+    float ffMean, nhP, ffFixed, logPMean, x1;
+    float dimMean, dimNorm, dimScale;
+    bool dim;      // the last analog's fallback score applies (x0 > x1)
+};
+
+__device__ void ScorerSetupQuad(ScorerQ& q, const hwpa_lane_model& m, int z, int a)
+{
+    const float log2pi = 1.8378770664f;
+    const float pi = 3.1415926536f;
+    const float sqrtHalfPi = hw_sqrtf(0.5f * pi);
+    const float bMean = hw_h2f(m.baseline.means[z]);
+    const float bVar = hw_h2f(m.baseline.vars[z]);
+    const float bSigma = hw_sqrtf(bVar);
+    const float normConst = log2pi / 2.0f;
+    q.x0 = bMean + bSigma * sqrtHalfPi;
+    q.nhB = -0.5f * (1.0f / bVar);
+    q.bgFixed = -0.5f * hw_cephes_logf(bVar) - normConst;
+    q.bgMean = bMean;
+    const float aMean = hw_h2f(m.analogs[a].means[z]);
+    const float aVar = hw_h2f(m.analogs[a].vars[z]);
+    const float aSigma = hw_sqrtf(aVar);
+    q.logPMean = hw_cephes_logf(aMean - bMean);
+    q.x1 = aMean - aSigma * sqrtHalfPi;
+    q.nhP = -0.5f * (1.0f / aVar);
+    q.ffFixed = -0.5f * hw_cephes_logf(aVar) - normConst;
+    q.ffMean = aMean;
+    // (the fallback's values; used by the last analog only)
+    const float eMean = 0.5f * (bMean + aMean);
+    float eVar = (1.0f / 6.0f) * (aMean - bMean);
+    eVar += bVar + aVar;
+    eVar *= 0.5f;
+    q.dimMean = eMean;
+    q.dimNorm = -0.5f * (log2pi + hw_cephes_logf(eVar));
+    q.dimScale = 0.5f / eVar;
+    q.dim = a == NA - 1 && !(q.x0 <= q.x1);
+}
+
+struct TransQ {    // a thread's part of TransVals
+    float b0, bu, bd;          // row B: candidates B, up_a, and the down states
+    float u0, uu[NA], ud;      // row up_a: candidates B, the up states, the down states
+    float f0, f1, d0, d1;      // rows full_a and down_a: candidates full_a, up_a
+};
+
+__global__ __launch_bounds__(256) void LabelQuadKernel(const int16_t* __restrict__ traces, int frames,
+                                                       const hwpa_lane_model* __restrict__ models,
+                                                       LabLaneState* state, uint16_t* __restrict__ tbAll, int tbFrames,
+                                                       int16_t* __restrict__ labels, int16_t* __restrict__ latentOut,
+                                                       float* __restrict__ score, TransVals T, float roiUpper,
+                                                       float roiLower)
+{
+    extern __shared__ uint32_t roiWords[];   // [(nroi + 15) / 16][LS], 2 bits per frame; a wave uses its own columns
+    const int lane = blockIdx.x;
+    const int a = threadIdx.x & 3;
+    const int z = threadIdx.x >> 2;
+    LabLaneState& st = state[lane];
+    const hwpa_lane_model& model = models[lane];
+    const int16_t* tr = traces + (size_t)lane * frames * LS + z;
+    uint16_t* tb = tbAll + ((size_t)lane * tbFrames * LS + z) * 4;   // [frame][ZMW][4]
+    const int nroi = frames + HWPA_VITERBI_LOOKBACK + HWPA_ROI_STITCH;
+    const int nlab = frames + HWPA_VITERBI_LOOKBACK;
+    const int nwords = (nroi + 15) / 16;
+
+#pragma unroll
+    for (int i = 0; i < NL; i += 4) latentOut[((size_t)lane * NL + i + a) * LS + z] = st.prevLat[i + a][z];
+
+    const float inv1 = 1.0f / hw_sqrtf(hw_h2f(st.oldModel.baseline.vars[z]));
+    const float inv2 = 1.0f / hw_sqrtf(hw_h2f(model.baseline.vars[z]));
+    // Frame k of the latent ++ chunk sequence, from a selected address (no branch).
+    const int seq = NL + frames;
+    auto rawAt = [&](int k) -> int {
+        const int16_t* p = (k < NL) ? &st.prevLat[k][z] : tr + (size_t)(k - NL) * LS;
+        return (int)*p;
+    };
+
+    // ROI forward pass: thread a compares frames 4a .. 4a + 3 of each 16-frame word with both
+    // thresholds (the sums of a frame depend on the frames around it only); the hysteresis
+    // then runs over the word's bits: r_k = r_{k-1} ? (m_k >= lower) : (m_k >= upper).
+    {
+        const float kS2 = 1.41421353816986083984375f;   // sqrt(2.0f)
+        const float kS3 = 1.73205077648162841796875f;   // sqrt(3.0f)
+        const float kR2 = 1.0f / kS2, kR3 = 1.0f / kS3;
+        uint32_t carry = st.roiBoundary[z] & 1u;
+        const int firstRaw = (int)st.latentTrc[z];
+        // Frames 16 w + 4 a - 1 .. + 5 (frame -1 is the one before the latent frames; frames
+        // past the sequence re-read its last one and are not used).
+        auto load = [&](int w, int (&dst)[7]) {
+#pragma unroll
+            for (int u = 0; u < 7; ++u) dst[u] = rawAt(min(max(16 * w + 4 * a - 1 + u, 0), seq - 1));
+        };
+        int cur[7], nxt[7];
+        load(0, cur);
+        for (int w = 0; w < nwords; ++w) {
+            load(w + 1, nxt);
+            float n[7];
+#pragma unroll
+            for (int u = 0; u < 7; ++u) {
+                const int k = 16 * w + 4 * a - 1 + u;
+                n[u] = (float)((k < 0) ? firstRaw : cur[u]) * ((k < NL) ? inv1 : inv2);
+            }
+            uint32_t up = 0, low = 0;
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const float a2 = n[u] + n[u + 1];
+                const float a3 = a2 + n[u + 2];
+                const float a4 = a3 + n[u + 3];
+                float mval = hw_maxf(n[u + 1], hw_div_by_const(a2, kS2, kR2));
+                mval = hw_maxf(mval, hw_div_by_const(a3, kS3, kR3));
+                mval = hw_maxf(mval, a4 * 0.5f);
+                const bool in = 16 * w + 4 * a + u < nroi;
+                up |= (in && mval >= roiUpper) ? 1u << (2 * u) : 0u;
+                low |= (in && mval >= roiLower) ? 1u << (2 * u) : 0u;
+            }
+            const uint32_t U = QuadOr(up << (8 * a)), L = QuadOr(low << (8 * a));
+            uint32_t R = 0;
+            if (roiUpper >= roiLower) {
+                // U implies L: r_k = u_k | (l_k & r_{k-1}) is the carry chain of one addition.
+                const uint32_t g = U << 1, pr = L << 1;
+                const uint32_t x = g | pr | 0x55555555u;
+                const uint32_t cin = (x + g + carry) ^ x ^ g;
+                R = (g | (pr & cin)) >> 1;
+                carry = (R >> 30) & 1u;
+            } else {
+#pragma unroll
+                for (int k = 0; k < 16; ++k) {
+                    carry = ((carry ? L : U) >> (2 * k)) & 1u;
+                    R |= carry << (2 * k);
+                }
+            }
+            if (a == 0) roiWords[w * LS + z] = R | (L << 1);
+#pragma unroll
+            for (int u = 0; u < 7; ++u) cur[u] = nxt[u];
+        }
+    }
+    // ROI backward pass, a word at a time (all four threads form the same word).  The words pass
+    // between lanes of one wave only, whose LDS and memory accesses stay in order: the fences keep
+    // the compiler from moving them.
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    {
+        uint32_t carry = 0;
+        for (int wi = nwords - 1; wi >= 0; --wi) {
+            const uint32_t v = hw_roi_backward_word(roiWords[wi * LS + z], &carry);
+            if (a == 0) roiWords[wi * LS + z] = v;
+        }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+
+    TransQ t;
+    t.b0 = T.bu[0][0];
+    t.bd = T.bd[0];
+    t.bu = a == 0 ? T.bu[0][1] : a == 1 ? T.bu[0][2] : a == 2 ? T.bu[0][3] : T.bu[0][4];
+    {
+        auto pick = [&](float v0, float v1, float v2, float v3) { return a == 0 ? v0 : a == 1 ? v1 : a == 2 ? v2 : v3; };
+        t.u0 = pick(T.bu[1][0], T.bu[2][0], T.bu[3][0], T.bu[4][0]);
+#pragma unroll
+        for (int p = 0; p < NA; ++p) t.uu[p] = pick(T.bu[1][1 + p], T.bu[2][1 + p], T.bu[3][1 + p], T.bu[4][1 + p]);
+        t.ud = pick(T.bd[1], T.bd[2], T.bd[3], T.bd[4]);
+        t.f0 = pick(T.fd[0][0], T.fd[1][0], T.fd[2][0], T.fd[3][0]);
+        t.f1 = pick(T.fd[0][1], T.fd[1][1], T.fd[2][1], T.fd[3][1]);
+        t.d0 = pick(T.fd[4][0], T.fd[5][0], T.fd[6][0], T.fd[7][0]);
+        t.d1 = pick(T.fd[4][1], T.fd[5][1], T.fd[6][1], T.fd[7][1]);
+    }
+    const uint32_t nibF = 4u * (uint32_t)a, nibU = nibF + 1u, nibD = nibF + 2u;
+
+    float lB, lF, lU, lD;
+    {
+        const float ninf = hw_u2f(0xff800000u);
+        const int lb = st.labelBoundary[z];
+        lB = lb == 0 ? 0.0f : ninf;
+        lF = lb == 1 + a ? 0.0f : ninf;
+        lU = lb == 5 + a ? 0.0f : ninf;
+        lD = lb == 9 + a ? 0.0f : ninf;
+    }
+    ScorerQ sc;
+    // One frame: Scores and Recur of LabelKernel.
+    auto step = [&](int f, float d, uint32_t rw) {
+        const float pen = RoiPen(rw, 2u * (uint32_t)(f & 15));
+        float y = d - sc.bgMean;
+        const float sB = (y * sc.nhB) * y + sc.bgFixed;
+        y = d - sc.ffMean;
+        const float sF = (y * sc.nhP) * y + sc.ffFixed;
+        const bool lowExt = d < sc.x0;
+        const float cap = lowExt ? sc.x0 : sc.x1;
+        const float fixedTerm = lowExt ? sc.nhB : sc.nhP;
+        const bool ext = lowExt || (d > sc.x1);
+        const float dc = d - cap;
+        float s = (ext ? fixedTerm * (dc * dc) : 0.0f) - sc.logPMean;
+        {
+            const float dm = d - sc.dimMean;
+            const float fb = sc.dimNorm - (dm * dm) * sc.dimScale;
+            s = sc.dim ? fb : s;
+        }
+        if (d > sc.ffMean) s = hw_minf(hw_minf(s, sF - 1.0f), 0.0f);
+
+        // Row B.  The running maximum over {B, up 0-3, down 0-3} with later candidates winning
+        // ties, a NaN candidate never winning and a NaN first one never replaced, equals: the
+        // (IEEE) maximum of the eight, the last of them that reaches it, taken if >= B's.
+        const float cB = (sB + t.b0) + lB;
+        const float cU = (sB + t.bu) + lU;
+        const float cD = (sB + t.bd) + lD;
+        float m8 = __builtin_fmaxf(cU, cD);
+        m8 = __builtin_fmaxf(m8, QuadF<kQuadXor1>(m8));
+        m8 = __builtin_fmaxf(m8, QuadF<kQuadXor2>(m8));
+        uint32_t code = (cU == m8) ? 1u + (uint32_t)a : 0u;
+        code = (cD == m8) ? 5u + (uint32_t)a : code;
+        code = QuadMaxU(code);
+        const bool takeB = m8 >= cB;
+        const float nB = takeB ? m8 : cB;
+        // candidate code -> nibble index: 0 the baseline, 1 + p up_p, 5 + p down_p
+        const uint32_t kB = takeB ? (4u * code - (code > 4u ? 18u : 3u)) : kNibB;
+
+        // Row up_a, candidate by candidate.
+        float mx = (s + t.u0) + lB;
+        uint32_t kU = kNibB;
+#pragma unroll
+        for (int p = 0; p < NA; ++p) {
+            const float v = (s + t.uu[p]) + QuadAt(lU, p);
+            const bool c = v >= mx;
+            mx = c ? v : mx;
+            kU = c ? 4u * (uint32_t)p + 1u : kU;
+        }
+        const float sd = s + t.ud;
+#pragma unroll
+        for (int p = 0; p < NA; ++p) {
+            const float v = sd + QuadAt(lD, p);
+            const bool c = v >= mx;
+            mx = c ? v : mx;
+            kU = c ? 4u * (uint32_t)p + 2u : kU;
+        }
+        // Rows full_a and down_a: candidates {full_a, up_a}.
+        const float fa = (sF + t.f0) + lF, fb = (sF + t.f1) + lU;
+        const bool cF = fb >= fa;
+        const float da = (s + t.d0) + lF, db = (s + t.d1) + lU;
+        const bool cDn = db >= da;
+        lF = (cF ? fb : fa) - pen;
+        lD = (cDn ? db : da) - pen;
+        lU = mx - pen;
+        lB = nB;
+        uint32_t w = cF ? nibU : nibF;
+        w |= kU << 4;
+        w |= (cDn ? nibU : nibF) << 8;
+        w |= kB << 12;
+        tb[(size_t)f * LS * 4 + a] = (uint16_t)w;
+    };
+    // Frames [f0, f1) of the sequence, four at a time when f0 is a multiple of 4 (so the four
+    // share an ROI word) with the next sixteen samples in flight: thread a holds frame 4 g + a of
+    // each group.
+    auto run = [&](int f0, int f1) {
+        const bool whole = (f0 & 3) == 0;
+        auto sample = [&](int g) { return rawAt(min(f0 + 4 * g + a, seq - 1)); };
+        int nx[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) nx[q] = sample(q);
+        int g = 0;
+        for (; whole && f0 + 16 * (g + 1) <= f1; ++g) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const float mine = (float)nx[q];
+                nx[q] = sample(4 * (g + 1) + q);
+                const int fq = f0 + 16 * g + 4 * q;
+                const uint32_t rw = roiWords[(fq >> 4) * LS + z];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) step(fq + u, QuadAt(mine, u), rw);
+            }
+        }
+        // The remainder, frame by frame (its samples are read by all four threads).
+        int f = f0 + 16 * g;
+        int raw = rawAt(min(f, seq - 1));
+#pragma unroll 1
+        for (; f < f1; ++f) {
+            const int next = rawAt(min(f + 1, seq - 1));
+            step(f, (float)raw, roiWords[(f >> 4) * LS + z]);
+            raw = next;
+        }
+    };
+    // The latent frames are scored with the previous chunk's model, the chunk and stitch frames
+    // with the current one; the log-likelihoods at the chunk's last frame are kept.
+    ScorerSetupQuad(sc, st.oldModel, z, a);
+    run(0, NL);
+    ScorerSetupQuad(sc, model, z, a);
+    run(NL, frames);
+    const float aB = lB, aF = lF, aU = lU, aD = lD;
+    run(frames, nlab);
+
+    // Normalise and propagate the end-state probabilities back over the stitch frames.
+    float pB, pF, pU, pD;
+    {
+        float all[NS];
+        all[0] = lB;
+#pragma unroll
+        for (int p = 0; p < NA; ++p) {
+            all[1 + p] = QuadAt(lF, p);
+            all[5 + p] = QuadAt(lU, p);
+            all[9 + p] = QuadAt(lD, p);
+        }
+        float mx = all[0];
+#pragma unroll
+        for (int i = 1; i < NS; ++i) mx = hw_maxf(all[i], mx);
+        pB = hw_cephes_expf(lB - mx);
+        pF = hw_cephes_expf(lF - mx);
+        pU = hw_cephes_expf(lU - mx);
+        pD = hw_cephes_expf(lD - mx);
+        float sum = 0.0f;
+        sum += pB;
+#pragma unroll
+        for (int p = 0; p < NA; ++p) sum += QuadAt(pF, p);
+#pragma unroll
+        for (int p = 0; p < NA; ++p) sum += QuadAt(pU, p);
+#pragma unroll
+        for (int p = 0; p < NA; ++p) sum += QuadAt(pD, p);
+        const float inv = 1 / sum;
+        pB *= inv;
+        pF *= inv;
+        pU *= inv;
+        pD *= inv;
+    }
+#pragma unroll 1
+    for (int i = nlab - 1; i > frames - 1; --i) {
+        // What each state passes to its predecessor, added in state order (a state's own sum
+        // gets +0 from the others, which leaves it as it is).
+        const uint32_t w = tb[(size_t)i * LS * 4 + a];
+        const uint32_t kB = (w >> 12) & 15u, kU = (w >> 4) & 15u, kF = w & 15u, kD = (w >> 8) & 15u;
+        float qU[NA];
+        uint32_t jU[NA];
+#pragma unroll
+        for (int p = 0; p < NA; ++p) {
+            qU[p] = QuadAt(pU, p);
+            jU[p] = QuadAtU(kU, p);
+        }
+        auto into = [&](uint32_t n, bool own) {
+            float v = 0.0f;
+            v += (kB == n) ? pB : 0.0f;
+            if (own) v += (kF == n) ? pF : 0.0f;
+#pragma unroll
+            for (int p = 0; p < NA; ++p) v += (jU[p] == n) ? qU[p] : 0.0f;
+            if (own) v += (kD == n) ? pD : 0.0f;
+            return v;
+        };
+        const float nB = into(kNibB, false), nF = into(nibF, true), nU = into(nibU, true), nD = into(nibD, false);
+        pB = nB;
+        pF = nF;
+        pU = nU;
+        pD = nD;
+    }
+    float maxProb = pB, sv = aB;
+    int anchorState = 0;
+    auto consider = [&](float p, float ll, int i) {
+        const bool cond = maxProb > p;
+        maxProb = cond ? maxProb : p;
+        sv = cond ? sv : ll;
+        anchorState = cond ? anchorState : i;
+    };
+#pragma unroll
+    for (int p = 0; p < NA; ++p) consider(QuadAt(pF, p), QuadAt(aF, p), 1 + p);
+#pragma unroll
+    for (int p = 0; p < NA; ++p) consider(QuadAt(pU, p), QuadAt(aU, p), 5 + p);
+#pragma unroll
+    for (int p = 0; p < NA; ++p) consider(QuadAt(pD, p), QuadAt(aD, p), 9 + p);
+    if (a == 0) score[(size_t)lane * LS + z] = sv;
+
+    // Traceback: thread a reads the whole 64-bit words of frames top - a - 4 q and writes their
+    // labels; every thread follows the path.
+    {
+        int16_t* lo = labels + (size_t)lane * frames * LS + z;
+        typedef uint32_t Word64 __attribute__((ext_vector_type(2), may_alias));
+        const Word64* tw = reinterpret_cast<const Word64*>(tb);   // [frame][ZMW]
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        uint32_t n = StateNib(anchorState);
+        auto word = [&](int top) { return tw[(size_t)max(top - a, 0) * LS]; };
+        Word64 nx[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) nx[q] = word(frames - 1 - 4 * q);
+        for (int top = frames - 1; top >= 0; top -= 16) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const Word64 w = nx[q];
+                nx[q] = word(top - 16 - 4 * q);
+                uint32_t mine = 0;
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    mine = (a == u) ? n : mine;
+                    const uint64_t v = (uint64_t)QuadAtU(w.x, u) | ((uint64_t)QuadAtU(w.y, u) << 32);
+                    n = (uint32_t)(v >> (4u * n)) & 15u;
+                }
+                const int f = top - 4 * q - a;
+                if (f >= 0) lo[(size_t)f * LS] = (int16_t)NibState(mine);
+            }
+        }
+    }
+
+    // Latent update
+    const int anchor = frames - NL;
+    const int fl = frames - 1;
+    int16_t lat[NL / 4];
+#pragma unroll
+    for (int i = 0; i < NL / 4; ++i) lat[i] = tr[(size_t)(anchor + 4 * i + a) * LS];
+#pragma unroll
+    for (int i = 0; i < NL / 4; ++i) st.prevLat[4 * i + a][z] = lat[i];
+    if (a == 0) {
+        st.roiBoundary[z] = (uint16_t)((roiWords[(fl >> 4) * LS + z] >> (2 * (fl & 15))) & 1u);
+        st.labelBoundary[z] = (int16_t)anchorState;
+        st.latentTrc[z] = tr[(size_t)(anchor - 1) * LS];
+        st.oldModel.baseline.means[z] = model.baseline.means[z];
+        st.oldModel.baseline.vars[z] = model.baseline.vars[z];
+        st.oldModel.baseline.weights[z] = model.baseline.weights[z];
+        st.oldModel.confidence[z] = model.confidence[z];
+    }
+    st.oldModel.analogs[a].means[z] = model.analogs[a].means[z];
+    st.oldModel.analogs[a].vars[z] = model.analogs[a].vars[z];
+    st.oldModel.analogs[a].weights[z] = model.analogs[a].weights[z];
+}
+
 __global__ __launch_bounds__(64) void LabelInitKernel(LabLaneState* state)
 {
     LabLaneState& st = state[blockIdx.x];
@@ -599,9 +1073,12 @@ int32_t LabelerCreate(const hwpa_config& cfg, uint32_t lanes, uint32_t max_frame
     l->lanes = lanes;
     l->maxFrames = max_frames;
     int32_t rc = DeviceAlloc((void**)&l->state, sizeof(LabLaneState) * lanes, "labeler state");
-    if (rc == HWPA_OK)
-        rc = DeviceAlloc((void**)&l->tb, (size_t)lanes * (max_frames + HWPA_VITERBI_LOOKBACK + NS) * LS * sizeof(uint32_t),
-                         "labeler traceback");
+    l->quad = lanes <= kQuadLanes;
+    if (rc == HWPA_OK) {
+        const size_t rows = max_frames + HWPA_VITERBI_LOOKBACK;
+        const size_t words = l->quad ? std::max<size_t>(rows + NS, 2 * rows) : rows + NS;
+        rc = DeviceAlloc((void**)&l->tb, (size_t)lanes * words * LS * sizeof(uint32_t), "labeler traceback");
+    }
     if (rc == HWPA_OK) {
         hipLaunchKernelGGL(LabelInitKernel, dim3(lanes), dim3(LS), 0, nullptr, l->state);
         rc = CheckLaunch("LabelInitKernel");
@@ -623,6 +1100,11 @@ void LabelerDestroy(LabelerDev* l)
     delete l;
 }
 
+void LabelerShare(LabelerDev* l, uint64_t lanes)
+{
+    l->quad = l->quad && lanes <= kQuadLanes;
+}
+
 int32_t LabelerRun(LabelerDev* l, const int16_t* traces, uint32_t frames, const hwpa_lane_model* models,
                    int16_t* labels, int16_t* latent_out, float* score, hipStream_t s)
 {
@@ -632,7 +1114,11 @@ int32_t LabelerRun(LabelerDev* l, const int16_t* traces, uint32_t frames, const 
         return Fail(HWPA_ERR_INVALID_ARG, "labeler_run: frames outside (24, max_frames]");
     const int nroi = (int)frames + HWPA_VITERBI_LOOKBACK + HWPA_ROI_STITCH;
     const size_t lds = (size_t)((nroi + 15) / 16) * LS * sizeof(uint32_t);
-    // Variants: frames per prefetched batch x registers held to 4 waves per SIMD.
+    // Variants: frames per prefetched batch x registers held to 4 waves per SIMD; 0 is the choice
+    // by size: four threads per ZMW for small pools (above), <16, 4> for 4,096 lanes and more of
+    // chunks up to 512 frames (4,096 x 512: 1.17 ms; <8, 1> 1.19, and <16, 1>, the earlier
+    // default, 1.25), else <8, 1> (1,024 x 512: 0.49 ms; <16, 4> 0.53, <16, 1> 0.50; 4,096 x 1024,
+    // where the ROI words in LDS limit the waves per SIMD anyway: 2.95 ms; <16, 4> 3.41).
 #define HWPA_LABEL_LAUNCH(PB, W)                                                                                   \
     hipLaunchKernelGGL((LabelKernel<PB, W>), dim3(l->lanes), dim3(LS), lds, s, traces, (int)frames, models,        \
                        l->state, l->tb, (int)(l->maxFrames + HWPA_VITERBI_LOOKBACK + NS), labels, latent_out,      \
@@ -641,7 +1127,17 @@ int32_t LabelerRun(LabelerDev* l, const int16_t* traces, uint32_t frames, const 
     case 1: HWPA_LABEL_LAUNCH(8, 1); break;
     case 2: HWPA_LABEL_LAUNCH(8, 4); break;
     case 3: HWPA_LABEL_LAUNCH(16, 4); break;
-    default: HWPA_LABEL_LAUNCH(16, 1); break;
+    default:
+        if (l->quad)
+            hipLaunchKernelGGL(LabelQuadKernel, dim3(l->lanes), dim3(4 * LS), lds, s, traces, (int)frames, models,
+                               l->state, reinterpret_cast<uint16_t*>(l->tb),
+                               (int)(l->maxFrames + HWPA_VITERBI_LOOKBACK), labels, latent_out, score, l->T,
+                               l->roiUpper, l->roiLower);
+        else if (l->lanes >= 4096 && frames <= 512)
+            HWPA_LABEL_LAUNCH(16, 4);
+        else
+            HWPA_LABEL_LAUNCH(8, 1);
+        break;
     }
 #undef HWPA_LABEL_LAUNCH
     return CheckLaunch("LabelKernel");

@@ -372,6 +372,46 @@ def test_labeler_bit_exact(H, O, T, gpu, label_variant, F):
         assert np.array_equal(H.to_numpy(d_score, np.float32, (L, 64)).view(np.uint32), o_score.view(np.uint32))
 
 
+@pytest.mark.parametrize("lanes,frames,thresholds", [(1, 25, (7.0, 2.0)), (3, 39, (7.0, 2.0)), (2, 130, (2.0, 7.0)),
+                                                     (2, 1029, (0.5, 0.25)), (768, 41, (7.0, 2.0)),
+                                                     (769, 41, (7.0, 2.0))])
+def test_labeler_small_pools_bit_exact(H, O, T, gpu, lanes, frames, thresholds):
+    """The default labeler of small pools (four threads per ZMW) at its edges: the shortest chunk,
+    frame counts that leave 1, 2 or 3 frames over a group of four, an upper ROI threshold below
+    the lower one, one lane, and the largest pool it takes and the next; degenerate models (NaN,
+    infinite and equal means, zero and huge variances) in some ZMWs."""
+    rng = np.random.default_rng(frames)
+    cfg = H.bench_config(512)
+    cfg.roi_upper_threshold, cfg.roi_lower_threshold = thresholds
+    tr = (rng.normal(0, 12, size=(3, lanes, frames, 64)) + 60.0 * (rng.random((3, lanes, frames, 64)) < 0.3))
+    tr = tr.round().astype(np.int16)
+    models = np.zeros(lanes, dtype=T.LANE_MODEL)
+    half = lambda v: np.asarray(v, dtype=np.float16).view(np.uint16)  # noqa: E731
+    models["baseline"]["means"] = half(rng.normal(0, 2, (lanes, 64)))
+    models["baseline"]["vars"] = half(rng.uniform(90, 160, (lanes, 64)))
+    for a, m in enumerate((180.0, 120.0, 80.0, 20.0)):
+        models["analogs"][:, a]["means"] = half(rng.normal(m, 5, (lanes, 64)))
+        models["analogs"][:, a]["vars"] = half(rng.uniform(200, 400, (lanes, 64)))
+    models["analogs"][:, 1]["means"][:, 7] = half(np.nan)
+    models["analogs"][:, 2]["vars"][:, 9] = half(0.0)
+    models["analogs"][:, 3]["means"][:, 11] = models["baseline"]["means"][:, 11]
+    models["analogs"][:, 0]["vars"][:, 13] = half(60000.0)
+    models["analogs"][:, 0]["means"][:, 15] = half(np.inf)
+    ol, gl = O.Labeler(cfg, lanes), H.Labeler(cfg, lanes, frames)
+    d_lab, d_lat = H.dev_bytes(lanes * frames * 64 * 2), H.dev_bytes(lanes * 24 * 64 * 2)
+    d_score = H.dev_bytes(lanes * 64 * 4)
+    for c in range(3):
+        o_lab, o_lat, o_score = ol.run(tr[c], models)
+        gl.run(_dev(H, tr[c]), frames, _dev(H, models), d_lab, d_lat, d_score)
+        g_lab = H.to_numpy(d_lab, np.int16, (lanes, frames, 64))
+        mism = np.argwhere(g_lab != o_lab)
+        assert len(mism) == 0, "chunk %d: %d label mismatches, first %s" % (c, len(mism), mism[:3].tolist())
+        assert np.array_equal(H.to_numpy(d_lat, np.int16, (lanes, 24, 64)), o_lat)
+        g_score = H.to_numpy(d_score, np.float32, (lanes, 64))
+        same = (g_score.view(np.uint32) == o_score.view(np.uint32)) | (np.isnan(g_score) & np.isnan(o_score))
+        assert same.all(), "chunk %d: %d scores differ" % (c, int((~same).sum()))
+
+
 @pytest.mark.parametrize("variant", [0, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12])
 @pytest.mark.parametrize("max_calls", [0, 480])
 def test_pulses_dense_boundaries_bit_exact(H, O, T, gpu, variant, max_calls):
