@@ -37,6 +37,36 @@ def test_baz_random_chunks_bit_exact(H, O, T, gpu, internal, zmws, mc):
         assert g_data == o_data, c
 
 
+@pytest.mark.parametrize("internal", [0, 1])
+def test_baz_row_edges_bit_exact(H, O, T, gpu, internal):
+    """Pulse counts 0 .. 63 over one lane's ZMWs and counts past the record capacity in the next
+    (every remainder of the 16-slot steps), ZMWs whose pulses are all rejected or all but the
+    last, and start gaps and widths around the overflow groups' limits (6, 13, 20 bits)."""
+    zmws, mc = 128, 64
+    rng = np.random.default_rng(9)
+    counts = np.concatenate([np.arange(64), rng.integers(60, 70, 64)]).astype(np.uint32)
+    p = np.zeros(zmws * mc, dtype=T.PULSE)
+    gaps = rng.choice(np.array([1, 62, 63, 64, 65, 8191, 8192, 8193, 1 << 20]), size=(zmws, mc), p=[.3] + [.0875] * 8)
+    p["start"] = (1000 + np.cumsum(gaps, axis=1)).astype(np.uint32).reshape(-1)
+    p["width"] = rng.choice(np.array([1, 2, 3, 63, 64, 8191, 8192, 65535]), size=zmws * mc)
+    p["mean_signal"], p["mid_signal"] = rng.integers(0, 65536, zmws * mc), rng.integers(0, 65536, zmws * mc)
+    p["max_signal"] = rng.integers(0, 300, zmws * mc)
+    p["signal_m2"] = rng.uniform(0, 9000, zmws * mc)
+    p["label"] = rng.integers(0, 4, zmws * mc)
+    p["is_reject"] = rng.integers(0, 2, zmws * mc)
+    p["is_reject"].reshape(zmws, mc)[[20, 70]] = 1
+    p["is_reject"].reshape(zmws, mc)[40, :39] = 1
+    enc = H.BazEncoder(zmws, internal=bool(internal))
+    last = np.zeros(zmws, dtype=np.uint64)
+    for c in range(2):
+        o_data, o_off, o_ev = O.baz_encode_batch(internal, p, counts, mc, last)
+        g_data, g_off, g_ev = _run(H, enc, p, counts, mc, len(o_data) + 64)
+        assert np.array_equal(g_off, o_off), c
+        assert np.array_equal(g_ev, o_ev), c
+        assert g_data == o_data, c
+        p["start"] += np.uint32(1 << 26)
+
+
 def test_baz_small_buffer_keeps_state(H, O, T, gpu):
     zmws, mc = 192, 12
     enc = H.BazEncoder(zmws)
