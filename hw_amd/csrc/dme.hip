@@ -306,7 +306,8 @@ struct EmExtra {
     const float* omap;        // EM_LEARNED: output map {off[6], scale[6], ...}
     uint8_t* fallback;        // EM_LEARNED: 1 = start rejected, model left for the plain EM
     float* diag;              // optional raw estimate [lane][HWPA_EM_DIAG_ROWS][64]
-    const uint32_t* active;   // optional: number of valid ZMWs; lanes at or beyond it exit
+    const uint32_t* active;   // optional: number of valid ZMWs; lanes at or beyond it exit, and the
+                              // last lane's missing ZMWs run as copies of its first one
     const uint8_t* laneSel;   // optional: only lanes whose 64 flags here are all set run
     float acceptConf;         // EM_LEARNED: minimum confidence to accept the capped EM
     float convTol;            // EM_LEARNED: relative log-likelihood convergence tolerance
@@ -343,7 +344,12 @@ __global__ __launch_bounds__(64, 3) void DmeEstimateKernel(const hwpa_lane_hist*
 {
     const int lane = blockIdx.x;
     const int z = threadIdx.x;
-    if (x.active && (uint32_t)lane * LS >= *x.active) return;
+    int zin = z;   // the ZMW whose inputs this thread reads
+    if (x.active) {
+        const uint32_t valid = *x.active;
+        if ((uint32_t)lane * LS >= valid) return;
+        if ((uint32_t)lane * LS + (uint32_t)z >= valid) zin = 0;
+    }
     if (x.laneSel && !__all(x.laneSel[(size_t)lane * LS + z] != 0)) return;
     bool gated = false;       // EM_LEARNED: the network's confidence sends this ZMW to the plain EM
     if (MODE == EM_LEARNED) {
@@ -369,8 +375,8 @@ __global__ __launch_bounds__(64, 3) void DmeEstimateKernel(const hwpa_lane_hist*
     const hwpa_baseliner_stats& bs = stats[lane];
     hwpa_lane_model& lm = models[lane];
 
-    HistView h{&lh, z, lh.low_bound[z], lh.bin_size[z]};
-    const uint32_t lowOut = lh.outlier_low[z], highOut = lh.outlier_high[z];
+    HistView h{&lh, zin, lh.low_bound[zin], lh.bin_size[zin]};
+    const uint32_t lowOut = lh.outlier_low[zin], highOut = lh.outlier_high[zin];
     int lastNz;
     float njSum;
     const uint32_t inRange = InRange(h, &lastNz, &njSum);
@@ -380,19 +386,19 @@ __global__ __launch_bounds__(64, 3) void DmeEstimateKernel(const hwpa_lane_hist*
     const float rpaSqSum = (rpa[0] * rpa[0] + rpa[2] * rpa[2]) + (rpa[1] * rpa[1] + rpa[3] * rpa[3]);
     const float rpaMin = hw_minf(hw_minf(rpa[0], rpa[1]), hw_minf(rpa[2], rpa[3]));
 
-    Model det = LoadModel(lm, z);
+    Model det = LoadModel(lm, zin);
     det.conf *= evolve;
 
     // PrelimEstimate (DmeEmHost.cpp:161-214)
     {
         Model w = det;
-        const float nBl = bs.baseline.m0[z];
-        const float total = bs.full.basic.m0[z];
+        const float nBl = bs.baseline.m0[zin];
+        const float total = bs.full.basic.m0[zin];
         const float blWeight = hw_maxf(nBl / total, 0.01f);
         const bool mask = nBl >= 3.0f;
-        float blVar = mask ? Variance(bs.baseline.m0[z], bs.baseline.m1[z], bs.baseline.m2[z]) : w.bl.var;
+        float blVar = mask ? Variance(bs.baseline.m0[zin], bs.baseline.m1[zin], bs.baseline.m2[zin]) : w.bl.var;
         blVar = hw_clampf(blVar, d.blVarMin, d.blVarMax);
-        const float blMean = mask ? (bs.baseline.m1[z] / bs.baseline.m0[z] + bs.baseline.offset[z]) : w.bl.mean;
+        const float blMean = mask ? (bs.baseline.m1[zin] / bs.baseline.m0[zin] + bs.baseline.offset[zin]) : w.bl.mean;
         const float scale = hw_sqrtf(blVar / w.bl.var);
 #pragma unroll
         for (int a = 0; a < NA; ++a) {
@@ -706,7 +712,7 @@ __global__ __launch_bounds__(64, 3) void DmeEstimateKernel(const hwpa_lane_hist*
             for (int j = 0; j < kRecurBlock; ++j) none |= (__all(cn[j] == 0u) ? 1u : 0u) << j;
             none = __builtin_amdgcn_readfirstlane(none);
             // Row of the next block's first bin (the last block's own is read when it is needed).
-            const uint16_t* ahead = &h.h->bin_count[min(b0 + kRecurBlock - 1, NB - kRecurBlock)][z];
+            const uint16_t* ahead = &h.h->bin_count[min(b0 + kRecurBlock - 1, NB - kRecurBlock)][zin];
             if (exAny != 0u || __popc(none) > 1) {
                 // Some component takes exp at every boundary, or bins are empty for the whole
                 // wave: both are left to wave-uniform branches.
@@ -897,7 +903,7 @@ __global__ __launch_bounds__(64, 3) void DmeEstimateKernel(const hwpa_lane_hist*
     }
     work.conf = conf;
     UpdateConf(d, det, work);
-    StoreModel(det, lm, z);
+    if (zin == z) StoreModel(det, lm, z);
 }
 
 // ---- fallback compaction for the learned start ---------------------------------
@@ -931,15 +937,6 @@ __device__ void ColStats(const hwpa_baseliner_stats& s, hwpa_baseliner_stats& d,
     ColStatAcc(s.background, d.background, sz, dz);
 }
 
-__device__ void ColHist(const hwpa_lane_hist& s, hwpa_lane_hist& d, int sz, int dz)
-{
-    d.low_bound[dz] = s.low_bound[sz];
-    d.bin_size[dz] = s.bin_size[sz];
-    d.outlier_low[dz] = s.outlier_low[sz];
-    d.outlier_high[dz] = s.outlier_high[sz];
-    for (int b = 0; b < NB; ++b) d.bin_count[b][dz] = s.bin_count[b][sz];
-}
-
 __device__ void ColModel(const hwpa_lane_model& s, hwpa_lane_model& d, int sz, int dz)
 {
     for (int a = 0; a < NA; ++a) {
@@ -965,7 +962,7 @@ __global__ __launch_bounds__(64) void FallbackCountKernel(const uint8_t* __restr
 __global__ __launch_bounds__(1024) void FallbackScanKernel(const uint32_t* __restrict__ cnt, uint32_t lanes,
                                                            uint32_t* __restrict__ off, uint32_t* __restrict__ total)
 {
-    __shared__ uint32_t part[1024], whole[1024];
+    __shared__ uint32_t part[16], whole[16];
     const uint32_t per = (lanes + 1023) / 1024;
     const uint32_t b0 = threadIdx.x * per, b1 = min(lanes, b0 + per);
     uint32_t s = 0, w = 0;
@@ -974,22 +971,32 @@ __global__ __launch_bounds__(1024) void FallbackScanKernel(const uint32_t* __res
         s += c == LS ? 0u : c;
         w += c == LS ? c : 0u;
     }
-    part[threadIdx.x] = s;
-    whole[threadIdx.x] = w;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        uint32_t run = 0, all = 0;
-        for (int i = 0; i < 1024; ++i) {
-            const uint32_t v = part[i];
-            part[i] = run;
-            run += v;
-            all += whole[i];
-        }
-        total[0] = run;
-        total[1] = run + all;
+    // Inclusive sums over the wave, then over the 16 waves.
+    const uint32_t t = threadIdx.x % 64, wv = threadIdx.x / 64;
+    uint32_t incl = s;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const uint32_t y = __shfl_up(incl, d, 64);
+        if (t >= (uint32_t)d) incl += y;
+        w += __shfl_xor(w, d, 64);
+    }
+    if (t == 63) {
+        part[wv] = incl;
+        whole[wv] = w;
     }
     __syncthreads();
-    uint32_t run = part[threadIdx.x];
+    uint32_t before = 0, sum = 0, all = 0;
+#pragma unroll
+    for (uint32_t k = 0; k < 16; ++k) {
+        before += k < wv ? part[k] : 0u;
+        sum += part[k];
+        all += whole[k];
+    }
+    if (threadIdx.x == 0) {
+        total[0] = sum;
+        total[1] = sum + all;
+    }
+    uint32_t run = before + incl - s;
     for (uint32_t i = b0; i < b1; ++i) {
         off[i] = run;
         const uint32_t c = cnt[i];
@@ -997,14 +1004,20 @@ __global__ __launch_bounds__(1024) void FallbackScanKernel(const uint32_t* __res
     }
 }
 
-__global__ __launch_bounds__(64) void FallbackGatherKernel(const uint8_t* __restrict__ fb, const uint32_t* __restrict__ off,
-                                                           const hwpa_lane_hist* __restrict__ hist,
-                                                           const hwpa_baseliner_stats* __restrict__ stats,
-                                                           const hwpa_lane_model* __restrict__ models,
-                                                           hwpa_lane_hist* cHist, hwpa_baseliner_stats* cStats,
-                                                           hwpa_lane_model* cModels, uint32_t* __restrict__ map)
+// One workgroup per lane: its four waves share the lane's bins, read 15 at a time (one wave
+// copying bin after bin took 75 us for 4,096 lanes, these 70: the rest is the traffic, rows
+// written in parts).
+constexpr int kGatherBatch = 15;
+static_assert(NB % (4 * kGatherBatch) == 0, "whole batches per wave");
+
+__global__ __launch_bounds__(256) void FallbackGatherKernel(const uint8_t* __restrict__ fb, const uint32_t* __restrict__ off,
+                                                            const hwpa_lane_hist* __restrict__ hist,
+                                                            const hwpa_baseliner_stats* __restrict__ stats,
+                                                            const hwpa_lane_model* __restrict__ models,
+                                                            hwpa_lane_hist* cHist, hwpa_baseliner_stats* cStats,
+                                                            hwpa_lane_model* cModels, uint32_t* __restrict__ map)
 {
-    const int lane = blockIdx.x, z = threadIdx.x;
+    const int lane = blockIdx.x, z = threadIdx.x % LS, w = threadIdx.x / LS;
     const bool f = fb[(size_t)lane * LS + z] != 0;
     const uint64_t m = __ballot(f);
     if (!f || m == ~0ull) return;
@@ -1012,26 +1025,26 @@ __global__ __launch_bounds__(64) void FallbackGatherKernel(const uint8_t* __rest
     const uint32_t pos = off[lane] + rank;
     const uint32_t cl = pos / LS;
     const int dz = (int)(pos % LS);
-    ColHist(hist[lane], cHist[cl], z, dz);
-    ColStats(stats[lane], cStats[cl], z, dz);
-    ColModel(models[lane], cModels[cl], z, dz);
-    map[pos] = (uint32_t)lane * LS + (uint32_t)z;
-}
-
-// Fills the unused slots of the last, partly filled compact lane with copies of
-// its first ZMW so that its EM behaves like a full lane.
-__global__ __launch_bounds__(64) void FallbackPadKernel(const uint32_t* __restrict__ total, hwpa_lane_hist* cHist,
-                                                        hwpa_baseliner_stats* cStats, hwpa_lane_model* cModels)
-{
-    const uint32_t t = *total;
-    const uint32_t used = t % LS;
-    if (used == 0) return;
-    const uint32_t cl = t / LS;
-    const int z = threadIdx.x;
-    if ((uint32_t)z < used) return;
-    ColHist(cHist[cl], cHist[cl], 0, z);
-    ColStats(cStats[cl], cStats[cl], 0, z);
-    ColModel(cModels[cl], cModels[cl], 0, z);
+    const hwpa_lane_hist& s = hist[lane];
+    hwpa_lane_hist& d = cHist[cl];
+    for (int b = w * (NB / 4); b < (w + 1) * (NB / 4); b += kGatherBatch) {
+        uint16_t c[kGatherBatch];
+#pragma unroll
+        for (int j = 0; j < kGatherBatch; ++j) c[j] = s.bin_count[b + j][z];
+#pragma unroll
+        for (int j = 0; j < kGatherBatch; ++j) d.bin_count[b + j][dz] = c[j];
+    }
+    if (w == 0) {
+        d.low_bound[dz] = s.low_bound[z];
+        d.bin_size[dz] = s.bin_size[z];
+        d.outlier_low[dz] = s.outlier_low[z];
+        d.outlier_high[dz] = s.outlier_high[z];
+        map[pos] = (uint32_t)lane * LS + (uint32_t)z;
+    } else if (w == 1) {
+        ColStats(stats[lane], cStats[cl], z, dz);
+    } else if (w == 2) {
+        ColModel(models[lane], cModels[cl], z, dz);
+    }
 }
 
 __global__ __launch_bounds__(64) void FallbackScatterKernel(const uint32_t* __restrict__ total,
@@ -1146,11 +1159,9 @@ int32_t DmeEstimateLearned(const hwpa_config& cfg, hwpa_initializer* mlp, Learne
     if ((rc = CheckLaunch("FallbackCountKernel")) != HWPA_OK) return rc;
     hipLaunchKernelGGL(FallbackScanKernel, dim3(1), dim3(1024), 0, s, w.cnt, lanes, w.off, w.total);
     if ((rc = CheckLaunch("FallbackScanKernel")) != HWPA_OK) return rc;
-    hipLaunchKernelGGL(FallbackGatherKernel, dim3(lanes), dim3(LS), 0, s, w.fallback, w.off, hist, stats, models,
+    hipLaunchKernelGGL(FallbackGatherKernel, dim3(lanes), dim3(4 * LS), 0, s, w.fallback, w.off, hist, stats, models,
                        w.cHist, w.cStats, w.cModels, w.map);
     if ((rc = CheckLaunch("FallbackGatherKernel")) != HWPA_OK) return rc;
-    hipLaunchKernelGGL(FallbackPadKernel, dim3(1), dim3(LS), 0, s, w.total, w.cHist, w.cStats, w.cModels);
-    if ((rc = CheckLaunch("FallbackPadKernel")) != HWPA_OK) return rc;
     EmExtra q{};
     q.laneSel = w.fallback;
     hipLaunchKernelGGL(DmeEstimateKernel<EM_PLAIN>, dim3(lanes), dim3(LS), 0, s, hist, stats, models,

@@ -114,6 +114,10 @@ struct LearnedWs {
 };
 int32_t LearnedWsAlloc(LearnedWs& w, uint32_t lanes);
 void LearnedWsFree(LearnedWs& w);
+// The same through the initialiser, which keeps one workspace between estimations; give it back
+// only when the stream that used it is idle.
+int32_t LearnedWsTake(hwpa_initializer* m, uint32_t lanes, LearnedWs& w);
+void LearnedWsGive(hwpa_initializer* m, LearnedWs& w);
 int32_t DmeEstimateLearned(const hwpa_config& cfg, hwpa_initializer* mlp, LearnedWs& w, const hwpa_lane_hist* hist,
                            const hwpa_baseliner_stats* stats, hwpa_lane_model* models, const int32_t model_fi[2],
                            const int32_t est_fi[2], uint32_t lanes, int32_t* d_iters, hipStream_t s);

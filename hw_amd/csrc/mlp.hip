@@ -18,6 +18,7 @@
 #include "internal.h"
 
 #include <cmath>
+#include <mutex>
 #include <vector>
 
 namespace hwpa {
@@ -416,9 +417,40 @@ struct hwpa_initializer {
     float* omap = nullptr;      // device {off[6], scale[6], w[8]}
     float omapHost[20] = {};
     float* kPart = nullptr;     // split-K partial weight gradients, kMaxSplit x MH x MH
+    // A learned-start workspace kept between estimations (LearnedWsTake), at most one.
+    std::mutex wsMutex;
+    LearnedWs ws;
 };
 
 namespace hwpa {
+
+// An estimation's workspace: the one the initialiser keeps if it is large enough and not in use,
+// else a new one.  Allocating and freeing its ten buffers on every call took 0.4 ms of a
+// 4,096-lane estimation's 4.1.
+int32_t LearnedWsTake(hwpa_initializer* m, uint32_t lanes, LearnedWs& w)
+{
+    {
+        std::lock_guard<std::mutex> g(m->wsMutex);
+        if (m->ws.lanes >= lanes) {
+            w = m->ws;
+            m->ws = LearnedWs{};
+            return HWPA_OK;
+        }
+    }
+    return LearnedWsAlloc(w, lanes);
+}
+
+// Gives a workspace back once nothing uses it; the larger of it and the kept one stays (up to
+// kKeepWsLanes lanes, 0.8 GB), the other is freed.
+void LearnedWsGive(hwpa_initializer* m, LearnedWs& w)
+{
+    constexpr uint32_t kKeepWsLanes = 16384;
+    if (w.lanes <= kKeepWsLanes) {
+        std::lock_guard<std::mutex> g(m->wsMutex);
+        if (w.lanes > m->ws.lanes) std::swap(w, m->ws);
+    }
+    LearnedWsFree(w);
+}
 
 static void FreeActs(hwpa_initializer* m)
 {
@@ -874,6 +906,7 @@ int32_t hwpa_initializer_destroy(hwpa_initializer* m)
     DeviceFree(m->lossDev);
     DeviceFree(m->omap);
     DeviceFree(m->kPart);
+    LearnedWsFree(m->ws);
     delete m;
     return HWPA_OK;
 }
