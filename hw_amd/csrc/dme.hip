@@ -564,9 +564,13 @@ __global__ __launch_bounds__(64, 3) void DmeEstimateKernel(const hwpa_lane_hist*
         // Whether every exponent of this iteration's restarts lies in [-8e6, 200] for all ZMWs
         // of the wave: then ExpBounded serves them (not the case only for degenerate models or
         // bounds: NaN, infinite, zero or negative variances).
+        // nanComp: this ZMW's components with a NaN parameter, whose density is NaN everywhere
+        // (a product as well as an exp of NaN), so they never need an exp per boundary.
         bool bounded = true;
+        uint32_t nanComp = 0;
 #pragma unroll
         for (int i = 0; i < 5; ++i) {
+            nanComp |= (hw_isnan(pref[i]) || hw_isnan(mu[i]) || hw_isnan(nhv[i]) ? 1u : 0u) << i;
             const float far = __builtin_fmaxf(hw_fabsf(h.lb - mu[i]), hw_fabsf(h.Start(NB) - mu[i]));
             bounded = bounded && nhv[i] <= 0.0f && (far * far) * nhv[i] >= -4e6f && pref[i] <= 80.0f && pref[i] >= -1e6f;
         }
@@ -617,8 +621,8 @@ __global__ __launch_bounds__(64, 3) void DmeEstimateKernel(const hwpa_lane_hist*
                 for (int i = 0; i < 5; ++i) {
                     const bool rec = (dd[i] >= FLT_MIN || dl[i] <= 0.0f) && dl[i] <= 80.0f;
                     const bool flat = tAt(x0, i) < kExpZeroBelow && tAt(x1, i) < kExpZeroBelow && x1 <= mu[i];
-                    if (!rec && flat) rr[i] = 0.0f;
-                    const bool ex = !rec && !flat;
+                    if (!rec && flat) rr[i] = 0.0f;   // (never for a NaN density)
+                    const bool ex = !rec && !flat && ((nanComp >> i) & 1u) == 0u;
                     exMask |= (ex ? 1u : 0u) << i;
                     exAny |= (__any(ex) ? 1u : 0u) << i;
                 }

@@ -302,14 +302,15 @@ def test_dme_estimate_recurrence_edge_paths_bit_exact(H, O, T, gpu):
     _eq_struct(H.to_numpy(d_models, T.LANE_MODEL, (L,)), o_models, "models")
 
 
-@pytest.mark.parametrize("shape", ["full_counters", "few_bins", "far_bounds"])
+@pytest.mark.parametrize("shape", ["full_counters", "few_bins", "far_bounds", "nan_models"])
 def test_dme_estimate_block_paths_bit_exact(H, O, T, gpu, shape):
     """The E-step's block forms against the oracle: counters whose sum passes 2^24 (every bin
     full), bins empty for a whole lane between occupied ones (branch per bin), and bins so wide
-    that the restarts' exponents leave the range of the unclamped exp."""
+    that the restarts' exponents leave the range of the unclamped exp, and ZMWs whose
+    start model is NaN (in which NaN equals NaN)."""
     L, F = 4, 512
     cfg, h, s, m = _em_case(H, O, T, L, F, 5)
-    h = h.copy()
+    h, m = h.copy(), m.copy()
     if shape == "full_counters":
         h["bin_count"][0] = 65535
         h["bin_count"][1, 100:] = 65000
@@ -321,6 +322,12 @@ def test_dme_estimate_block_paths_bit_exact(H, O, T, gpu, shape):
         h["bin_count"][1, 120:] = 0
         h["bin_count"][2, :20] = 0
         h["bin_count"][0:3, 18] += 150
+    elif shape == "nan_models":
+        nan = np.float16(np.nan).view(np.uint16)
+        m["baseline"]["means"][0, 5] = nan
+        m["analogs"][:, 2]["means"][1, 9] = nan
+        m["analogs"]["vars"][2, :, 3] = nan
+        m["baseline"]["vars"][3, 60] = nan
     else:
         h["bin_size"][0:2, 5::16] *= np.float32(3e3)
         h["low_bound"][1, 7::16] = np.float32(-3e5)
@@ -331,7 +338,11 @@ def test_dme_estimate_block_paths_bit_exact(H, O, T, gpu, shape):
     H.dme_estimate(cfg, _dev(H, h), _dev(H, s), d_models, mfi, efi, L, d_iters)
     iters = H.to_numpy(d_iters, np.int32, (L,))
     assert list(iters) == [diag[l].iterations_run for l in range(L)]
-    _eq_struct(H.to_numpy(d_models, T.LANE_MODEL, (L,)), o_models, "models")
+    g_models = H.to_numpy(d_models, T.LANE_MODEL, (L,))
+    for f in (g_models, o_models):
+        w = f.view(np.uint16)
+        w[(w & 0x7fff) > 0x7c00] = 0x7e00
+    _eq_struct(g_models, o_models, "models")
 
 
 @pytest.fixture(params=[0, 1, 2, 3])
