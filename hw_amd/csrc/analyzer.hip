@@ -81,6 +81,7 @@ using namespace hwpa;
 struct hwpa_analyzer {
     hwpa_config cfg;
     uint32_t poolId, lanes, frames;
+    uint32_t sideBySide = 0;   // lanes of all pools of the batch this one belongs to
     int32_t nextFrame = 0;
     uint32_t baselinerLatency = 0, dmeDelay = 0;
     bool fullEstimation = false;   // DynamicEstimate: a full estimation has occurred
@@ -205,13 +206,14 @@ static int32_t DmeAddBatch(hwpa_analyzer* a, int32_t first_frame)
             const int32_t mfi[2] = {a->modelFi.lo, a->modelFi.hi};
             const int32_t efi[2] = {a->histFi.lo, a->histFi.hi};
             if (a->mlp && a->cfg.learned_init) {
-                rc = DmeEstimateLearned(a->cfg, a->mlp, a->lws, a->dHist, a->dAgg, a->dModels, mfi, efi, L, a->dIters, s);
+                rc = DmeEstimateLearned(a->cfg, a->mlp, a->lws, a->dHist, a->dAgg, a->dModels, mfi, efi, L, a->dIters, s,
+                                        a->sideBySide);
                 a->ranLearned = true;
                 a->plan |= kPlanLearned;
             } else {
                 const bool cap = a->capX != nullptr;
                 rc = DmeEstimate(a->cfg, a->dHist, a->dAgg, a->dModels, mfi, efi, L, a->dIters, s,
-                                 cap ? a->dDiag : nullptr);
+                                 cap ? a->dDiag : nullptr, a->sideBySide);
                 if (rc == HWPA_OK && cap) rc = MlpFeatures(a->dHist, L, a->capX, s);
                 if (rc == HWPA_OK && cap)
                     rc = MlpTargets(a->dHist, a->dDiag, L, a->capMinConf, a->capT, a->capValid, s);
@@ -752,7 +754,10 @@ int32_t hwpa_batch_create(uint32_t n_pools, const uint32_t* pool_ids, const uint
     }
     uint64_t allLanes = 0;
     for (auto* a : b->pools) allLanes += a->lanes;
-    for (auto* a : b->pools) LabelerShare(a->lab, allLanes);
+    for (auto* a : b->pools) {
+        LabelerShare(a->lab, allLanes);
+        a->sideBySide = (uint32_t)std::min<uint64_t>(allLanes, UINT32_MAX);
+    }
     b->joins.assign(n_pools, nullptr);
     bool ok = hipStreamCreate(&b->master) == hipSuccess;
     ok = ok && hipEventCreateWithFlags(&b->fork, hipEventDisableTiming) == hipSuccess;

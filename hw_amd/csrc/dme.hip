@@ -13,6 +13,7 @@
 
 #include "internal.h"
 
+#include <algorithm>
 #include <cfloat>
 #include <mutex>
 
@@ -336,8 +337,9 @@ __device__ __forceinline__ float ExpBounded(float t)
     return hw_ldexpf(hw_exp_poly(r), (int)kf);
 }
 
-template <int MODE>
-__global__ __launch_bounds__(64, 3) void DmeEstimateKernel(const hwpa_lane_hist* __restrict__ hists,
+// MINW: waves per SIMD the registers allow (EmWavesPerSimd).
+template <int MODE, int MINW>
+__global__ __launch_bounds__(64, MINW) void DmeEstimateKernel(const hwpa_lane_hist* __restrict__ hists,
                                                         const hwpa_baseliner_stats* __restrict__ stats,
                                                         hwpa_lane_model* models, int32_t* iters, DmeDevCfg d,
                                                         float evolve, EmExtra x)
@@ -1081,18 +1083,46 @@ static float EvolveFactor(const DmeDevCfg& d, const int32_t model_fi[2], const i
     return hw_dexp2f(-hw_fabsf(tDiff) / hl);
 }
 
+// Waves per SIMD for a launch of `lanes` waves on 1,024 SIMDs.  Lanes take about equally
+// long, so what counts is the number of rounds.  Up to 2,048 lanes two waves per SIMD are all
+// there are, and the registers of 2 spill nothing (2,048 lanes, start-up estimate: 1.47 ms; held to
+// 3 waves 1.59, to 4 1.87); 3,073 to 4,096 lanes fit one round of 4 (4,096: 2.68 ms; 3 waves, whose
+// second round is a third full, 3.03); beyond, 3 is the best (32,768 lanes in a running pool: 12.7
+// ms; 4 13.2, 2 15.0; 8,192: 4.99; 5.35, 5.53), and between 2,049 and 3,072 its round suffices.
+// Pools that run side by side (one batch) share the registers, so their lanes count together (six
+// pools of 365 to 2,048 lanes in one graph: 7.1 ms a step, 7.5 with each pool's own choice).
+static int EmWavesPerSimd(uint32_t lanes)
+{
+    constexpr uint32_t kSimds = 1024;
+    return lanes <= 2 * kSimds ? 2 : (lanes > 3 * kSimds && lanes <= 4 * kSimds) ? 4 : 3;
+}
+
+template <int MODE>
+static int32_t EmLaunch(int waves, uint32_t lanes, hipStream_t s, const hwpa_lane_hist* hist,
+                        const hwpa_baseliner_stats* stats, hwpa_lane_model* models, int32_t* iters, const DmeDevCfg& d,
+                        float evolve, const EmExtra& x)
+{
+#define HWPA_EM_LAUNCH(W)                                                                                             \
+    hipLaunchKernelGGL((DmeEstimateKernel<MODE, W>), dim3(lanes), dim3(LS), 0, s, hist, stats, models, iters, d, evolve, x)
+    switch (waves) {
+    case 2: HWPA_EM_LAUNCH(2); break;
+    case 4: HWPA_EM_LAUNCH(4); break;
+    default: HWPA_EM_LAUNCH(3); break;
+    }
+#undef HWPA_EM_LAUNCH
+    return CheckLaunch("DmeEstimateKernel");
+}
+
 int32_t DmeEstimate(const hwpa_config& cfg, const hwpa_lane_hist* hist, const hwpa_baseliner_stats* stats,
                     hwpa_lane_model* models, const int32_t model_fi[2], const int32_t est_fi[2], uint32_t lanes,
-                    int32_t* d_iters, hipStream_t s, float* diag)
+                    int32_t* d_iters, hipStream_t s, float* diag, uint32_t sideBySide)
 {
     if (!hist || !stats || !models || lanes == 0) return Fail(HWPA_ERR_INVALID_ARG, "dme_estimate: bad argument");
     const DmeDevCfg d = MakeDevCfg(cfg);
     const float evolve = EvolveFactor(d, model_fi, est_fi);
     EmExtra x{};
     x.diag = diag;
-    hipLaunchKernelGGL(DmeEstimateKernel<EM_PLAIN>, dim3(lanes), dim3(LS), 0, s, hist, stats, models, d_iters, d,
-                       evolve, x);
-    return CheckLaunch("DmeEstimateKernel");
+    return EmLaunch<EM_PLAIN>(EmWavesPerSimd(std::max(lanes, sideBySide)), lanes, s, hist, stats, models, d_iters, d, evolve, x);
 }
 
 void LearnedWsFree(LearnedWs& w)
@@ -1138,7 +1168,8 @@ int32_t LearnedWsAlloc(LearnedWs& w, uint32_t lanes)
 
 int32_t DmeEstimateLearned(const hwpa_config& cfg, hwpa_initializer* mlp, LearnedWs& w, const hwpa_lane_hist* hist,
                            const hwpa_baseliner_stats* stats, hwpa_lane_model* models, const int32_t model_fi[2],
-                           const int32_t est_fi[2], uint32_t lanes, int32_t* d_iters, hipStream_t s)
+                           const int32_t est_fi[2], uint32_t lanes, int32_t* d_iters, hipStream_t s,
+                           uint32_t sideBySide)
 {
     if (!mlp || !hist || !stats || !models || lanes == 0 || lanes > w.lanes)
         return Fail(HWPA_ERR_INVALID_ARG, "dme_estimate_learned: bad argument");
@@ -1156,9 +1187,8 @@ int32_t DmeEstimateLearned(const hwpa_config& cfg, hwpa_initializer* mlp, Learne
     x.iterLimit = (int32_t)cfg.learned_em_iteration_limit;
     x.gateLogit = MlpGateLogit(cfg.learned_gate_threshold);
     x.laneMinConf = (int32_t)cfg.learned_lane_min_confident;
-    hipLaunchKernelGGL(DmeEstimateKernel<EM_LEARNED>, dim3(lanes), dim3(LS), 0, s, hist, stats, models, d_iters, d,
-                       evolve, x);
-    if ((rc = CheckLaunch("DmeEstimateKernel")) != HWPA_OK) return rc;
+    const int waves = EmWavesPerSimd(std::max(lanes, sideBySide));
+    if ((rc = EmLaunch<EM_LEARNED>(waves, lanes, s, hist, stats, models, d_iters, d, evolve, x)) != HWPA_OK) return rc;
     hipLaunchKernelGGL(FallbackCountKernel, dim3(lanes), dim3(LS), 0, s, w.fallback, w.cnt);
     if ((rc = CheckLaunch("FallbackCountKernel")) != HWPA_OK) return rc;
     hipLaunchKernelGGL(FallbackScanKernel, dim3(1), dim3(1024), 0, s, w.cnt, lanes, w.off, w.total);
@@ -1168,14 +1198,12 @@ int32_t DmeEstimateLearned(const hwpa_config& cfg, hwpa_initializer* mlp, Learne
     if ((rc = CheckLaunch("FallbackGatherKernel")) != HWPA_OK) return rc;
     EmExtra q{};
     q.laneSel = w.fallback;
-    hipLaunchKernelGGL(DmeEstimateKernel<EM_PLAIN>, dim3(lanes), dim3(LS), 0, s, hist, stats, models,
-                       static_cast<int32_t*>(nullptr), d, evolve, q);
-    if ((rc = CheckLaunch("DmeEstimateKernel")) != HWPA_OK) return rc;
+    if ((rc = EmLaunch<EM_PLAIN>(waves, lanes, s, hist, stats, models, nullptr, d, evolve, q)) != HWPA_OK) return rc;
+    // How many of these waves have work is known on the device only; it is seldom all of them.
     EmExtra p{};
     p.active = w.total;
-    hipLaunchKernelGGL(DmeEstimateKernel<EM_PLAIN>, dim3(lanes), dim3(LS), 0, s, w.cHist, w.cStats, w.cModels, w.cIters,
-                       d, evolve, p);
-    if ((rc = CheckLaunch("DmeEstimateKernel")) != HWPA_OK) return rc;
+    rc = EmLaunch<EM_PLAIN>(std::min(waves, 3), lanes, s, w.cHist, w.cStats, w.cModels, w.cIters, d, evolve, p);
+    if (rc != HWPA_OK) return rc;
     hipLaunchKernelGGL(FallbackScatterKernel, dim3(lanes), dim3(LS), 0, s, w.total, w.map, w.cModels, models);
     return CheckLaunch("FallbackScatterKernel");
 }

@@ -93,9 +93,10 @@ int32_t HistAddVariant(int32_t variant, hwpa_lane_hist* hist, void* edge, const 
 
 int32_t DmeInitModels(const hwpa_config& cfg, const hwpa_baseliner_stats* stats, hwpa_lane_model* models,
                       uint32_t lanes, hipStream_t s);
+// sideBySide: lanes of all the pools that run at the same time (0: this one's alone).
 int32_t DmeEstimate(const hwpa_config& cfg, const hwpa_lane_hist* hist, const hwpa_baseliner_stats* stats,
                     hwpa_lane_model* models, const int32_t model_fi[2], const int32_t est_fi[2], uint32_t lanes,
-                    int32_t* d_iters, hipStream_t s, float* diag = nullptr);
+                    int32_t* d_iters, hipStream_t s, float* diag = nullptr, uint32_t sideBySide = 0);
 
 // Learned start of the EM: network input/output and fallback compaction buffers
 // for up to `lanes` lanes.
@@ -120,7 +121,8 @@ int32_t LearnedWsTake(hwpa_initializer* m, uint32_t lanes, LearnedWs& w);
 void LearnedWsGive(hwpa_initializer* m, LearnedWs& w);
 int32_t DmeEstimateLearned(const hwpa_config& cfg, hwpa_initializer* mlp, LearnedWs& w, const hwpa_lane_hist* hist,
                            const hwpa_baseliner_stats* stats, hwpa_lane_model* models, const int32_t model_fi[2],
-                           const int32_t est_fi[2], uint32_t lanes, int32_t* d_iters, hipStream_t s);
+                           const int32_t est_fi[2], uint32_t lanes, int32_t* d_iters, hipStream_t s,
+                           uint32_t sideBySide = 0);
 int32_t MlpFeatures(const hwpa_lane_hist* hist, uint32_t lanes, uint16_t* x, hipStream_t s);
 // Network outputs for every ZMW of `lanes` lane histograms (features computed in the kernel).
 int32_t MlpForwardFromHist(const hwpa_initializer* m, const hwpa_lane_hist* hist, uint32_t lanes, float* y,
