@@ -337,22 +337,54 @@ __device__ __forceinline__ float ExpBounded(float t)
     return hw_ldexpf(hw_exp_poly(r), (int)kf);
 }
 
-// MINW: waves per SIMD the registers allow (EmWavesPerSimd).
-template <int MODE, int MINW>
-__global__ __launch_bounds__(64, MINW) void DmeEstimateKernel(const hwpa_lane_hist* __restrict__ hists,
+// The E-step of small pools (QUAD): four threads per ZMW, a workgroup of four waves per lane, for
+// launches that leave SIMDs without a wave.  The boundaries are taken in groups of four blocks:
+// thread u forms block u's densities, bin probabilities, logs and weights, leaves them in LDS in
+// boundary order, and then carries a quarter of the fourteen running sums over the group's 40
+// boundaries: its analog's two, one of the baseline's four, and the probability's or the
+// log-likelihood's.  Each sum is formed in the same order from the same terms, so the bits stay.
+// What counts is the instructions of one wave, which issues one in four cycles: 131 thousand
+// against 314 (and 14 thousand LDS accesses).  48 lanes in a running pool: 0.60 against 0.97 ms;
+// start-up estimate: 48 lanes 0.74 against 1.27 ms, 256 lanes 0.75 against 1.33, 384 lanes (two
+// rounds) 1.38 against 1.37.
+constexpr int kQuadGroup = 4 * kRecurBlock;
+constexpr int kQuadRow = kQuadGroup + 4;   // a row holds the boundary before the group too; 16-byte rows
+enum { QR_D = 0, QR_F = 5, QR_G, QR_DEV, QR_W, QR_WD, QR_P, QR_N, QR_LG, QR_ROWS };
+constexpr int kQuadZmw = QR_ROWS * kQuadRow;
+
+// Value of quad thread P, and of the thread before in the quad (thread 0 gets thread 3's).
+template <int P>
+__device__ __forceinline__ float EmQuadAt(float v)
+{
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), P * 0x55, 0xf, 0xf, true));
+}
+__device__ __forceinline__ float EmQuadPrev(float v)
+{
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x93, 0xf, 0xf, true));   // [3, 0, 1, 2]
+}
+
+// MINW: waves per SIMD the registers allow (EmWavesPerSimd).  QUAD: see above.
+template <int MODE, int MINW, bool QUAD = false>
+__global__ __launch_bounds__(QUAD ? 4 * LS : LS, MINW) void DmeEstimateKernel(const hwpa_lane_hist* __restrict__ hists,
                                                         const hwpa_baseliner_stats* __restrict__ stats,
                                                         hwpa_lane_model* models, int32_t* iters, DmeDevCfg d,
                                                         float evolve, EmExtra x)
 {
     const int lane = blockIdx.x;
-    const int z = threadIdx.x;
+    const int z = QUAD ? threadIdx.x >> 2 : threadIdx.x;
+    const int u = QUAD ? threadIdx.x & 3 : 0;   // place in the quad; place 0 writes the results
+    // Votes over the lane's 64 ZMWs.
+    auto laneAll = [](bool v) -> bool { return QUAD ? __syncthreads_and(v ? 1 : 0) != 0 : (bool)__all(v); };
+    auto laneCount = [&](bool v) -> int {
+        return QUAD ? __syncthreads_count(v && u == 0 ? 1 : 0) : (int)__popcll(__ballot(v));
+    };
     int zin = z;   // the ZMW whose inputs this thread reads
     if (x.active) {
         const uint32_t valid = *x.active;
         if ((uint32_t)lane * LS >= valid) return;
         if ((uint32_t)lane * LS + (uint32_t)z >= valid) zin = 0;
     }
-    if (x.laneSel && !__all(x.laneSel[(size_t)lane * LS + z] != 0)) return;
+    if (x.laneSel && !laneAll(x.laneSel[(size_t)lane * LS + z] != 0)) return;
     bool gated = false;       // EM_LEARNED: the network's confidence sends this ZMW to the plain EM
     if (MODE == EM_LEARNED) {
         // Confidence gate: a ZMW below it takes no capped iteration of its own (it still
@@ -361,17 +393,20 @@ __global__ __launch_bounds__(64, MINW) void DmeEstimateKernel(const hwpa_lane_hi
         // would cost the whole lane for those few).  A lane gated whole leaves its models
         // as they are, as every rejected ZMW does, and stops here.
         gated = !(x.init[((size_t)lane * LS + z) * HWPA_MLP_OUT + 11] >= x.gateLogit);
-        if (__popcll(__ballot(!gated)) < (uint32_t)x.laneMinConf) gated = true;
-        if (__all(gated)) {
+        if ((uint32_t)laneCount(!gated) < (uint32_t)x.laneMinConf) gated = true;
+        if (laneAll(gated)) {
             x.fallback[(size_t)lane * LS + z] = 1;
-            if (z == 0 && iters) iters[lane] = 0;
+            if (threadIdx.x == 0 && iters) iters[lane] = 0;
             return;
         }
     }
     // Tables of the E-step's log / reciprocal of bin probabilities, one entry per thread.
     __shared__ float sRc[HW_LOGTAB_N], sLc[HW_LOGTAB_N];
     static_assert(HW_LOGTAB_N == LS, "one table entry per thread");
-    hw_logtab_entry(z, &sRc[z], &sLc[z]);
+    if (threadIdx.x < LS) hw_logtab_entry(threadIdx.x, &sRc[threadIdx.x], &sLc[threadIdx.x]);
+    __shared__ __align__(16) float sQuad[QUAD ? LS * kQuadZmw : 1];
+    __shared__ __align__(16) float sOnes[QUAD ? kQuadRow : 1];
+    if (QUAD && threadIdx.x < (unsigned)kQuadRow) sOnes[threadIdx.x] = 1.0f;
     __syncthreads();
     const hwpa_lane_hist& lh = hists[lane];
     const hwpa_baseliner_stats& bs = stats[lane];
@@ -577,6 +612,188 @@ __global__ __launch_bounds__(64, MINW) void DmeEstimateKernel(const hwpa_lane_hi
             bounded = bounded && nhv[i] <= 0.0f && (far * far) * nhv[i] >= -4e6f && pref[i] <= 80.0f && pref[i] >= -1e6f;
         }
         bounded = __all(bounded);
+        float maxMu = mu[0];
+#pragma unroll
+        for (int k = 1; k < 5; ++k) maxMu = hw_maxf(maxMu, mu[k]);
+        if constexpr (QUAD) {
+            float* q = sQuad + z * kQuadZmw;
+            auto row = [&](int r) -> float* { return q + r * kQuadRow; };
+            // This thread's sums: own[c] += A B for its analog's two, the baseline's one and (0)
+            // the probability's or (1) the log-likelihood's.
+            float own = 0.0f, ownX = 0.0f, base = 0.0f, acc = 0.0f;
+            const float* baseA = u < 2 ? row(QR_D) : u == 2 ? row(QR_W) : row(QR_WD);
+            const float* baseB = u == 0 ? row(QR_F) : u == 1 ? row(QR_G) : row(QR_DEV);
+            const float* accA = u == 0 ? row(QR_P) : row(QR_N);
+            const float* accB = u == 0 ? sOnes : row(QR_LG);
+            const float* ownD = row(QR_D + 1 + u);
+            float bpC = 0.0f, fC = 0.0f, d0C = 0.0f;   // of the boundary before the group
+            float fFirst = 0.0f;                       // weight of the bin before the thread's block
+            row(QR_D + 1 + u)[0] = 0.0f;
+            if (u == 0) row(QR_D)[0] = 0.0f;
+            auto count = [&](int c) -> uint32_t {      // of the bin before boundary c
+                return (uint32_t)lh.bin_count[min(max(c - 1, 0), NB - 1)][zin];
+            };
+            uint32_t cn[kRecurBlock];
+#pragma unroll
+            for (int j = 0; j < kRecurBlock; ++j) cn[j] = count(kRecurBlock * u + j);
+            int cLast = NB, at = NB % kQuadGroup + 1;   // the last boundary taken, its place in the rows
+#pragma unroll 1
+            for (int g0 = 0; g0 <= NB; g0 += kQuadGroup) {
+                if (g0 > 0) {
+                    const float tol = hw_ldexpf(EmQuadAt<0>(acc), -27);
+                    const bool tail = lastNz < g0 - 1 && h.Start(g0 - 1) > maxMu && h.bs * bpC < tol && binProbMin < tol;
+                    if (__all(tail)) {
+                        cLast = g0 - 1;
+                        at = 0;
+                        break;
+                    }
+                }
+                const int c0 = g0 + kRecurBlock * u;   // the thread's first boundary
+                uint32_t exMask = 0;
+                {
+                    const float x0 = h.Start(c0), x1 = h.Start(c0 + kRecurBlock);
+#pragma unroll
+                    for (int i = 0; i < 5; ++i) {
+                        const float y0 = x0 - mu[i];
+                        const float t0 = hw_fmaf(y0 * y0, nhv[i], pref[i]);
+                        const float dl = nbs[i] * hw_fmaf(2.0f, y0, h.bs);
+                        if (bounded) {
+                            dd[i] = ExpBounded(t0);
+                            rr[i] = ExpBounded(dl);
+                        } else {
+                            dd[i] = hw_expf(t0);
+                            rr[i] = hw_expf(dl);
+                        }
+                        const bool rec = (dd[i] >= FLT_MIN || dl <= 0.0f) && dl <= 80.0f;
+                        const bool flat = t0 < kExpZeroBelow && tAt(x1, i) < kExpZeroBelow && x1 <= mu[i];
+                        if ((!rec && flat) || t0 < kExpZeroBelow) rr[i] = 0.0f;   // +0 from here on, or an exp below
+                        exMask |= (!rec && !flat && ((nanComp >> i) & 1u) == 0u && c0 < NB ? 1u : 0u) << i;
+                    }
+                }
+                const bool anyEx = __any(exMask != 0u);
+                float bp[kRecurBlock], f[kRecurBlock], d0[kRecurBlock];
+#pragma unroll
+                for (int j = 0; j < kRecurBlock; ++j) {
+                    if (j > 0) {
+#pragma unroll
+                        for (int i = 0; i < 5; ++i) {
+                            dd[i] = dd[i] * rr[i];
+                            rr[i] = rr[i] * qq[i];
+                        }
+                        if (anyEx) {
+                            const float x = h.Start(c0 + j);
+#pragma unroll
+                            for (int i = 0; i < 5; ++i)
+                                if ((exMask >> i) & 1u) dd[i] = hw_expf(tAt(x, i));
+                        }
+                    }
+                    const bool in = c0 + j <= NB;
+                    bp[j] = in ? Sum5Tree(dd) : 0.0f;
+                    d0[j] = in ? dd[0] : 0.0f;
+#pragma unroll
+                    for (int i = 0; i < 5; ++i) row(QR_D + i)[kRecurBlock * u + j + 1] = in ? dd[i] : 0.0f;
+                }
+                const float bpB = EmQuadPrev(bp[kRecurBlock - 1]);
+                float bpPrev = u == 0 ? bpC : bpB;
+                bpC = EmQuadAt<3>(bp[kRecurBlock - 1]);
+#pragma unroll
+                for (int j = 0; j < kRecurBlock; ++j) {
+                    const bool in = c0 + j <= NB && (j > 0 || c0 > 0);   // (no bin before boundary 0)
+                    const float binp = hw_max_pos(halfBin * (bpPrev + bp[j]), binProbMin);
+                    bpPrev = bp[j];
+                    const float nj = in ? (float)cn[j] : 0.0f;
+                    float lg, rcp;
+                    hw_log_rcp_tab(binp, sRc, sLc, &lg, &rcp);
+                    f[j] = nj * rcp;
+                    const int p = kRecurBlock * u + j;
+                    row(QR_P)[p] = in ? binp : 0.0f;
+                    row(QR_N)[p] = nj;
+                    row(QR_LG)[p] = lg;
+                    cn[j] = count(c0 + kQuadGroup + j);
+                }
+                const float fB = EmQuadPrev(f[kRecurBlock - 1]), d0B = EmQuadPrev(d0[kRecurBlock - 1]);
+                float fPrev = u == 0 ? fC : fB, d0Prev = u == 0 ? d0C : d0B;
+                fC = EmQuadAt<3>(f[kRecurBlock - 1]);
+                d0C = EmQuadAt<3>(d0[kRecurBlock - 1]);
+                fFirst = f[0];
+#pragma unroll
+                for (int j = 0; j < kRecurBlock; ++j) {
+                    // Terms of boundary c0 + j - 1.
+                    const bool in = c0 + j <= NB;
+                    const float x = h.Start(c0 + j - 1);
+                    const float F = in ? fPrev + f[j] : 0.0f;
+                    const float dev = x - piv;
+                    const float w = d0Prev * F;
+                    const int p = kRecurBlock * u + j;
+                    row(QR_F)[p] = F;
+                    row(QR_G)[p] = x * F;
+                    row(QR_DEV)[p] = dev;
+                    row(QR_W)[p] = w;
+                    row(QR_WD)[p] = w * dev;
+                    fPrev = f[j];
+                    d0Prev = d0[j];
+                }
+                // The rows pass between lanes of one wave only; its LDS accesses stay in order.
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll 2
+                for (int p = 0; p < kQuadGroup; p += 4) {
+                    const float4 vd = *reinterpret_cast<const float4*>(ownD + p);
+                    const float4 vF = *reinterpret_cast<const float4*>(row(QR_F) + p);
+                    const float4 vG = *reinterpret_cast<const float4*>(row(QR_G) + p);
+                    const float4 a = *reinterpret_cast<const float4*>(baseA + p);
+                    const float4 b = *reinterpret_cast<const float4*>(baseB + p);
+                    const float4 ea = *reinterpret_cast<const float4*>(accA + p);
+                    const float4 eb = *reinterpret_cast<const float4*>(accB + p);
+                    own = hw_fmaf(vd.x, vF.x, own);
+                    own = hw_fmaf(vd.y, vF.y, own);
+                    own = hw_fmaf(vd.z, vF.z, own);
+                    own = hw_fmaf(vd.w, vF.w, own);
+                    ownX = hw_fmaf(vd.x, vG.x, ownX);
+                    ownX = hw_fmaf(vd.y, vG.y, ownX);
+                    ownX = hw_fmaf(vd.z, vG.z, ownX);
+                    ownX = hw_fmaf(vd.w, vG.w, ownX);
+                    base = hw_fmaf(a.x, b.x, base);
+                    base = hw_fmaf(a.y, b.y, base);
+                    base = hw_fmaf(a.z, b.z, base);
+                    base = hw_fmaf(a.w, b.w, base);
+                    acc = hw_fmaf(ea.x, eb.x, acc);
+                    acc = hw_fmaf(ea.y, eb.y, acc);
+                    acc = hw_fmaf(ea.z, eb.z, acc);
+                    acc = hw_fmaf(ea.w, eb.w, acc);
+                }
+                if (g0 + kQuadGroup <= NB) {
+                    row(QR_D + 1 + u)[0] = ownD[kQuadGroup];
+                    if (u == 0) row(QR_D)[0] = row(QR_D)[kQuadGroup];
+                }
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            }
+            // The last boundary's own terms: its weight is that of the bin before it.
+            {
+                constexpr int kLastThread = NB % kQuadGroup / kRecurBlock;
+                const float F = cLast == NB ? EmQuadAt<kLastThread>(fFirst) : fC;
+                const float x = h.Start(cLast);
+                const float G = x * F, dev = x - piv;
+                const float dOwn = ownD[at], dBl = row(QR_D)[at];
+                const float w = dBl * F;
+                own = hw_fmaf(dOwn, F, own);
+                ownX = hw_fmaf(dOwn, G, ownX);
+                base = hw_fmaf(u < 2 ? dBl : u == 2 ? w : w * dev, u == 0 ? F : u == 1 ? G : dev, base);
+            }
+            ci[0] = EmQuadAt<0>(base);
+            mom1[0] = EmQuadAt<1>(base);
+            q1 = EmQuadAt<2>(base);
+            q2 = EmQuadAt<3>(base);
+            ci[1] = EmQuadAt<0>(own);
+            ci[2] = EmQuadAt<1>(own);
+            ci[3] = EmQuadAt<2>(own);
+            ci[4] = EmQuadAt<3>(own);
+            mom1[1] = EmQuadAt<0>(ownX);
+            mom1[2] = EmQuadAt<1>(ownX);
+            mom1[3] = EmQuadAt<2>(ownX);
+            mom1[4] = EmQuadAt<3>(ownX);
+            probSum = EmQuadAt<0>(acc);
+            wps = EmQuadAt<1>(acc);
+        } else {
         uint32_t exMask = 0;   // this ZMW's components that take exp at every boundary of the block
         uint32_t exAny = 0;    // the same for any ZMW of the wave
         bool zeroBl = false;   // the baseline density is +0 through the block for the whole wave
@@ -685,9 +902,6 @@ __global__ __launch_bounds__(64, MINW) void DmeEstimateKernel(const hwpa_lane_hi
         // an ulp of probSum, so adding them would leave it unchanged, and every other sum
         // of those boundaries is an exact zero (empty bins).  The result equals the full
         // pass bit for bit.
-        float maxMu = mu[0];
-#pragma unroll
-        for (int k = 1; k < 5; ++k) maxMu = hw_maxf(maxMu, mu[k]);
         // Counts of a block's bins b0 - 1 .. b0 + 8, each read again for the next block as
         // soon as it has been used, so its load is in flight over a whole block.
         uint32_t cn[kRecurBlock];
@@ -772,6 +986,7 @@ __global__ __launch_bounds__(64, MINW) void DmeEstimateKernel(const hwpa_lane_hi
             }
         }
         gather(h.Start(cLast), fPrev, true);
+        }
         const float q0 = ci[0];
 #pragma unroll
         for (int m = 0; m < 5; ++m) {
@@ -798,7 +1013,7 @@ __global__ __launch_bounds__(64, MINW) void DmeEstimateKernel(const hwpa_lane_hi
         converged = converged || conv;
         // Lane-wide early exit (DmeEmHost.cpp:485)
         const bool done = converged || (status != HWPA_ZS_OK) || gated;
-        if (!d.iterToLimit && __all(done)) break;
+        if (!d.iterToLimit && laneAll(done)) break;
 
         // ---- M-step
         float c[5];
@@ -840,7 +1055,7 @@ __global__ __launch_bounds__(64, MINW) void DmeEstimateKernel(const hwpa_lane_hi
         for (int a = 0; a < NA; ++a) var[a + 1] = Covar(d, d.cv[a] * d.cv[a], mu[a + 1], var[0]);
     }
     if (!converged) status |= HWPA_ZS_NO_CONVERGE;
-    if (z == 0 && iters) iters[lane] = it;
+    if (threadIdx.x == 0 && iters) iters[lane] = it;
 
     work.bl.w = rhoEst[0];
     work.bl.mean = muEst[0];
@@ -890,7 +1105,7 @@ __global__ __launch_bounds__(64, MINW) void DmeEstimateKernel(const hwpa_lane_hi
     }
     conf = hw_minf(hw_maxf(0.0f, conf), 1.0f);
     conf = (conf >= d.successThresh) ? conf : 0.0f;
-    if (x.diag) {
+    if (x.diag && u == 0) {
         float* dg = x.diag + (size_t)lane * HWPA_EM_DIAG_ROWS * LS + z;
 #pragma unroll
         for (int k = 0; k < 5; ++k) {
@@ -904,12 +1119,12 @@ __global__ __launch_bounds__(64, MINW) void DmeEstimateKernel(const hwpa_lane_hi
     }
     if (MODE == EM_LEARNED) {
         const bool accept = !gated && converged && status == HWPA_ZS_OK && conf >= x.acceptConf;
-        x.fallback[(size_t)lane * LS + z] = accept ? 0 : 1;
+        if (u == 0) x.fallback[(size_t)lane * LS + z] = accept ? 0 : 1;
         if (!accept) return;
     }
     work.conf = conf;
     UpdateConf(d, det, work);
-    if (zin == z) StoreModel(det, lm, z);
+    if (zin == z && u == 0) StoreModel(det, lm, z);
 }
 
 // ---- fallback compaction for the learned start ---------------------------------
@@ -1083,6 +1298,10 @@ static float EvolveFactor(const DmeDevCfg& d, const int32_t model_fi[2], const i
     return hw_dexp2f(-hw_fabsf(tDiff) / hl);
 }
 
+// Up to one lane per CU, four threads per ZMW (the kernel's QUAD form; its rows take 143 KB of
+// LDS, so a second lane on the CU waits for the first).
+constexpr uint32_t kEmQuadLanes = 256;
+
 // Waves per SIMD for a launch of `lanes` waves on 1,024 SIMDs.  Lanes take about equally
 // long, so what counts is the number of rounds.  Up to 2,048 lanes two waves per SIMD are all
 // there are, and the registers of 2 spill nothing (2,048 lanes, start-up estimate: 1.47 ms; held to
@@ -1094,6 +1313,7 @@ static float EvolveFactor(const DmeDevCfg& d, const int32_t model_fi[2], const i
 static int EmWavesPerSimd(uint32_t lanes)
 {
     constexpr uint32_t kSimds = 1024;
+    if (lanes <= kEmQuadLanes) return 1;
     return lanes <= 2 * kSimds ? 2 : (lanes > 3 * kSimds && lanes <= 4 * kSimds) ? 4 : 3;
 }
 
@@ -1102,6 +1322,11 @@ static int32_t EmLaunch(int waves, uint32_t lanes, hipStream_t s, const hwpa_lan
                         const hwpa_baseliner_stats* stats, hwpa_lane_model* models, int32_t* iters, const DmeDevCfg& d,
                         float evolve, const EmExtra& x)
 {
+    if (waves == 1) {
+        hipLaunchKernelGGL((DmeEstimateKernel<MODE, 1, true>), dim3(lanes), dim3(4 * LS), 0, s, hist, stats, models,
+                           iters, d, evolve, x);
+        return CheckLaunch("DmeEstimateKernel");
+    }
 #define HWPA_EM_LAUNCH(W)                                                                                             \
     hipLaunchKernelGGL((DmeEstimateKernel<MODE, W>), dim3(lanes), dim3(LS), 0, s, hist, stats, models, iters, d, evolve, x)
     switch (waves) {

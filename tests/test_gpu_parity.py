@@ -345,6 +345,37 @@ def test_dme_estimate_block_paths_bit_exact(H, O, T, gpu, shape):
     _eq_struct(g_models, o_models, "models")
 
 
+@pytest.mark.parametrize("lanes", [1, 256, 257, 2049, 3073, 4097])
+@pytest.mark.parametrize("seed", [3, 5])
+def test_dme_estimate_forms_bit_exact(H, O, T, gpu, lanes, seed):
+    """Each form of the EM kernel (chosen by the number of lanes) at the edges of its range, on
+    the lanes of one case repeated, the edge paths of the recurrence, sparse and far-off
+    histograms and a NaN start model among them."""
+    L, F = 5, 512
+    cfg, h, s, m = _em_case(H, O, T, L, F, seed, tg=dict(snr_lo=3.0, snr_hi=20.0, empty_fraction=0.1))
+    h, m = h.copy(), m.copy()
+    bs = h["bin_size"].copy()
+    h["low_bound"][1, 0::2] -= 100.0 * bs[1, 0::2]
+    h["bin_size"][1, 1::4] *= 8.0
+    h["bin_count"][2, 10:40] = 0
+    h["bin_count"][2, 130:] = 0
+    h["bin_size"][3, 5::16] *= np.float32(3e3)
+    m["analogs"][:, 2]["means"][4, 9] = np.float16(np.nan).view(np.uint16)
+    mfi, efi = (512, 1024), (1024, 1536)
+    o_models, diag = O.dme_estimate(cfg, h, s, m, mfi, efi, want_diag=True, form="mirror")
+    at = np.arange(lanes) % L
+    d_models = _dev(H, m[at])
+    d_iters = H.dev_bytes(lanes * 4)
+    H.dme_estimate(cfg, _dev(H, h[at]), _dev(H, s[at]), d_models, mfi, efi, lanes, d_iters)
+    iters = H.to_numpy(d_iters, np.int32, (lanes,))
+    assert list(iters) == [diag[l].iterations_run for l in at]
+    g, o = H.to_numpy(d_models, T.LANE_MODEL, (lanes,)), o_models[at]
+    for f in (g, o):
+        w = f.view(np.uint16)
+        w[(w & 0x7fff) > 0x7c00] = 0x7e00
+    _eq_struct(g, o, "models")
+
+
 @pytest.fixture(params=[0, 1, 2, 3])
 def label_variant(request, H):
     """Every autotuner variant of the labeler (16 or 8 frames per batch, registers
