@@ -81,7 +81,9 @@ using namespace hwpa;
 struct hwpa_analyzer {
     hwpa_config cfg;
     uint32_t poolId, lanes, frames;
-    uint32_t sideBySide = 0;   // lanes of all pools of the batch this one belongs to
+    // Lanes taken to be at work at the same time: those of all pools of the batch this one belongs
+    // to, or three pools like this one (pools run on their own streams, several at a time).
+    uint32_t sideBySide = 0;
     int32_t nextFrame = 0;
     uint32_t baselinerLatency = 0, dmeDelay = 0;
     bool fullEstimation = false;   // DynamicEstimate: a full estimation has occurred
@@ -261,6 +263,7 @@ int32_t hwpa_analyzer_create(uint32_t pool_id, uint32_t lanes, uint32_t frames, 
     a->poolId = pool_id;
     a->lanes = lanes;
     a->frames = frames;
+    a->sideBySide = (uint32_t)std::min<uint64_t>(3ull * lanes, UINT32_MAX);
     a->baselinerLatency = BaselinerStartupLatency(*cfg);
     const uint32_t cpe = (std::max(cfg->min_frames_for_estimate, 1u) + frames - 1) / frames;
     a->dmeDelay = (pool_id % cpe) * frames;

@@ -1302,19 +1302,24 @@ static float EvolveFactor(const DmeDevCfg& d, const int32_t model_fi[2], const i
 // LDS, so a second lane on the CU waits for the first).
 constexpr uint32_t kEmQuadLanes = 256;
 
-// Waves per SIMD for a launch of `lanes` waves on 1,024 SIMDs.  Lanes take about equally
-// long, so what counts is the number of rounds.  Up to 2,048 lanes two waves per SIMD are all
-// there are, and the registers of 2 spill nothing (2,048 lanes, start-up estimate: 1.47 ms; held to
-// 3 waves 1.59, to 4 1.87); 3,073 to 4,096 lanes fit one round of 4 (4,096: 2.68 ms; 3 waves, whose
-// second round is a third full, 3.03); beyond, 3 is the best (32,768 lanes in a running pool: 12.7
-// ms; 4 13.2, 2 15.0; 8,192: 4.99; 5.35, 5.53), and between 2,049 and 3,072 its round suffices.
-// Pools that run side by side (one batch) share the registers, so their lanes count together (six
-// pools of 365 to 2,048 lanes in one graph: 7.1 ms a step, 7.5 with each pool's own choice).
-static int EmWavesPerSimd(uint32_t lanes)
+// Waves per SIMD for a launch of `lanes` lanes on 1,024 SIMDs (1: four threads per ZMW).  Lanes
+// take about equally long, so what counts is the number of rounds.  Up to 2,048 lanes two waves per
+// SIMD are all there are, and the registers of 2 spill nothing (2,048 lanes, start-up estimate:
+// 1.47 ms; held to 3 waves 1.59, to 4 1.87); 3,073 to 4,096 lanes fit one round of 4 (4,096: 2.68
+// ms; 3 waves, whose second round is a third full, 3.03); beyond, 3 is the best (32,768 lanes in a
+// running pool: 12.7 ms; 4 13.2, 2 15.0; 8,192: 4.99; 5.35, 5.53), and between 2,049 and 3,072 its
+// round suffices.  Pools that run side by side share the SIMDs (sideBySide, their lanes together):
+// there a launch with fewer waves per SIMD keeps others out, and 3 is the choice past 2,048 (six
+// pools of 365 to 2,048 lanes in one graph: 7.1 ms a step, 7.5 with each pool's own choice; three
+// pools of 2,000 lanes on their streams: 1.71 ms a chunk against 1.82).  Four threads per ZMW pay up
+// to three such pools of 256 lanes (200 lanes each: 0.53 ms a chunk against 0.56).
+static int EmWavesPerSimd(uint32_t lanes, uint32_t sideBySide)
 {
     constexpr uint32_t kSimds = 1024;
-    if (lanes <= kEmQuadLanes) return 1;
-    return lanes <= 2 * kSimds ? 2 : (lanes > 3 * kSimds && lanes <= 4 * kSimds) ? 4 : 3;
+    const uint32_t all = std::max(lanes, sideBySide);
+    if (lanes <= kEmQuadLanes && all <= 3 * kEmQuadLanes) return 1;
+    if (all <= 2 * kSimds) return 2;
+    return (sideBySide == 0 && lanes > 3 * kSimds && lanes <= 4 * kSimds) ? 4 : 3;
 }
 
 template <int MODE>
@@ -1347,7 +1352,7 @@ int32_t DmeEstimate(const hwpa_config& cfg, const hwpa_lane_hist* hist, const hw
     const float evolve = EvolveFactor(d, model_fi, est_fi);
     EmExtra x{};
     x.diag = diag;
-    return EmLaunch<EM_PLAIN>(EmWavesPerSimd(std::max(lanes, sideBySide)), lanes, s, hist, stats, models, d_iters, d, evolve, x);
+    return EmLaunch<EM_PLAIN>(EmWavesPerSimd(lanes, sideBySide), lanes, s, hist, stats, models, d_iters, d, evolve, x);
 }
 
 void LearnedWsFree(LearnedWs& w)
@@ -1412,7 +1417,7 @@ int32_t DmeEstimateLearned(const hwpa_config& cfg, hwpa_initializer* mlp, Learne
     x.iterLimit = (int32_t)cfg.learned_em_iteration_limit;
     x.gateLogit = MlpGateLogit(cfg.learned_gate_threshold);
     x.laneMinConf = (int32_t)cfg.learned_lane_min_confident;
-    const int waves = EmWavesPerSimd(std::max(lanes, sideBySide));
+    const int waves = EmWavesPerSimd(lanes, sideBySide);
     if ((rc = EmLaunch<EM_LEARNED>(waves, lanes, s, hist, stats, models, d_iters, d, evolve, x)) != HWPA_OK) return rc;
     hipLaunchKernelGGL(FallbackCountKernel, dim3(lanes), dim3(LS), 0, s, w.fallback, w.cnt);
     if ((rc = CheckLaunch("FallbackCountKernel")) != HWPA_OK) return rc;

@@ -93,7 +93,7 @@ int32_t HistAddVariant(int32_t variant, hwpa_lane_hist* hist, void* edge, const 
 
 int32_t DmeInitModels(const hwpa_config& cfg, const hwpa_baseliner_stats* stats, hwpa_lane_model* models,
                       uint32_t lanes, hipStream_t s);
-// sideBySide: lanes of all the pools that run at the same time (0: this one's alone).
+// sideBySide: lanes taken to be at work at the same time, this launch's included (0: its own).
 int32_t DmeEstimate(const hwpa_config& cfg, const hwpa_lane_hist* hist, const hwpa_baseliner_stats* stats,
                     hwpa_lane_model* models, const int32_t model_fi[2], const int32_t est_fi[2], uint32_t lanes,
                     int32_t* d_iters, hipStream_t s, float* diag = nullptr, uint32_t sideBySide = 0);

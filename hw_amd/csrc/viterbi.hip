@@ -49,12 +49,12 @@ struct LabelerDev {
 
 // Pools of at most this many lanes are labeled by four threads per ZMW (LabelQuadKernel).  It
 // issues 1.5 times the instructions of LabelKernel, in waves 2.6 times shorter, so it wins until
-// its waves fill the chip's issue slots (512 frames, quad against one thread per ZMW): 16 lanes
+// its waves fill the chip's issue slots (512 frames, quad against one thread per ZMW: 16 lanes
 // 0.20 against 0.50 ms, 512 lanes 0.32 against 0.52, 1,024 lanes 0.55 against 0.54, 4,096 lanes
-// 1.9 against 1.2.  Pools that run side by side fill the chip together, so they count together
-// (six pools of 365 to 2,048 lanes in one graph: 7.1 ms a step, 7.3 with the two below 768 lanes
-// on four threads).
-constexpr uint32_t kQuadLanes = 768;
+// 1.9 against 1.2; three pools of 300 lanes on their streams: 0.67 against 0.70 ms a chunk, of 600
+// lanes 0.87 against 0.84).  Pools of one batch count together (six pools of 365 to 2,048 lanes in
+// one graph: 7.1 ms a step, 7.3 with the two smallest on four threads).
+constexpr uint32_t kQuadLanes = 512;
 
 // nhB = -1/(2 var_B), nhP = -1/(2 var_a): the reference's -0.5f * y * invVar * y
 // equals (y * (-0.5f * invVar)) * y bit for bit (scaling by -0.5 is exact here).

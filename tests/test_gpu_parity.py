@@ -415,8 +415,8 @@ def test_labeler_bit_exact(H, O, T, gpu, label_variant, F):
 
 
 @pytest.mark.parametrize("lanes,frames,thresholds", [(1, 25, (7.0, 2.0)), (3, 39, (7.0, 2.0)), (2, 130, (2.0, 7.0)),
-                                                     (2, 1029, (0.5, 0.25)), (768, 41, (7.0, 2.0)),
-                                                     (769, 41, (7.0, 2.0))])
+                                                     (2, 1029, (0.5, 0.25)), (512, 41, (7.0, 2.0)),
+                                                     (513, 41, (7.0, 2.0))])
 def test_labeler_small_pools_bit_exact(H, O, T, gpu, lanes, frames, thresholds):
     """The default labeler of small pools (four threads per ZMW) at its edges: the shortest chunk,
     frame counts that leave 1, 2 or 3 frames over a group of four, an upper ROI threshold below
