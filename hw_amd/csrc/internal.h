@@ -127,8 +127,6 @@ int32_t MlpFeatures(const hwpa_lane_hist* hist, uint32_t lanes, uint16_t* x, hip
 // Network outputs for every ZMW of `lanes` lane histograms (features computed in the kernel).
 int32_t MlpForwardFromHist(const hwpa_initializer* m, const hwpa_lane_hist* hist, uint32_t lanes, float* y,
                            hipStream_t s);
-int32_t MlpForward(const hwpa_initializer* m, const uint16_t* x, uint32_t rows, float* y, uint16_t* h1, uint16_t* h2,
-                   hipStream_t s);
 const float* MlpOutputMap(const hwpa_initializer* m);  // device {off[6], scale[6], w[8]}
 // Logit of the learned gate's probability threshold (host): the network's confidence
 // output is compared with it; a threshold of 0 lets every ZMW through.

@@ -7,16 +7,13 @@
 // A bf16 mirror of the whole vector feeds the matrix cores; biases are added
 // in fp32 from the master copy.
 //
-// One generic GEMM kernel serves every layer and every gradient:
-//   C[m][n] = sum_k A[m][k] * B[k][n]
-// with element strides for A and B (so transposed operands need no copies),
-// a 64x64 tile per 256-thread workgroup, one 32x32 sub-tile per wave and
-// v_mfma_f32_32x32x16_bf16 over k in steps of 16.  Operand lanes: lane l
+// Every product is v_mfma_f32_32x32x16_bf16 over k in steps of 16.  Operand lanes: lane l
 // supplies A[l%32][k0+8(l/32)+j] and B[k0+8(l/32)+j][l%32], j = 0..7; the 16
 // accumulators of lane l hold C[8(i/4)+4(l/32)+i%4][l%32].
 
 #include "internal.h"
 
+#include <algorithm>
 #include <cmath>
 #include <mutex>
 #include <vector>
@@ -36,163 +33,11 @@ constexpr size_t OFF_B3 = OFF_W3 + (size_t)MO * MH;
 constexpr size_t NPARAM = OFF_B3 + MO;
 static_assert(NPARAM == HWPA_MLP_PARAMS, "parameter count");
 
-enum { EPI_F32 = 0, EPI_BIAS_F32 = 1, EPI_BIAS_RELU_BF16 = 2, EPI_MASK_BF16 = 3 };
-
-struct GemmArgs {
-    const uint16_t* A;
-    int64_t a_m, a_k;
-    const uint16_t* B;
-    int64_t b_k, b_n;
-    int32_t M, N, K;
-    const float* bias;
-    const uint16_t* mask;
-    int64_t mk_m, mk_n;
-    float* Cf;
-    uint16_t* Cb;
-    int64_t c_m, c_n;
-    // Split-K (EPI_F32 only): slice ks of kSplit covers k in [ks * kSlice,
-    // (ks + 1) * kSlice) and writes its partial product at Cf + ks * sliceStride.
-    int32_t kSplit, kSlice;
-    int64_t sliceStride;
-};
-
-template <bool CONTIG>
-__device__ __forceinline__ bf16x8 LoadK(const uint16_t* __restrict__ p, bool valid, int64_t off, int k,
-                                        int64_t sk, int K)
-{
-    if (CONTIG && valid && k + 8 <= K) {
-        const uint4 q = *reinterpret_cast<const uint4*>(p + off + k);
-        return __builtin_bit_cast(bf16x8, q);
-    }
-    uint32_t w[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const int k0 = k + 2 * j, k1 = k0 + 1;
-        const uint32_t lo = (valid && k0 < K) ? p[off + (int64_t)k0 * sk] : 0u;
-        const uint32_t hi = (valid && k1 < K) ? p[off + (int64_t)k1 * sk] : 0u;
-        w[j] = lo | (hi << 16);
-    }
-    const uint4 q = make_uint4(w[0], w[1], w[2], w[3]);
-    return __builtin_bit_cast(bf16x8, q);
-}
-
 __device__ __forceinline__ bool PositiveBf16(uint16_t b) { return b != 0 && (b & 0x8000u) == 0; }
 
-template <bool AK, bool BK, int EPI>
-__global__ __launch_bounds__(256) void GemmKernel(GemmArgs g, uint32_t nTiles, uint32_t tiles)
+__device__ __forceinline__ bf16x8 LoadRow8(const uint16_t* __restrict__ p)
 {
-    const uint32_t tile = blockIdx.x % tiles, ks = blockIdx.x / tiles;
-    const int mt = (int)(tile / nTiles), nt = (int)(tile % nTiles);
-    const int wave = threadIdx.x >> 6, l = threadIdx.x & 63;
-    const int m0 = mt * 64 + (wave >> 1) * 32, n0 = nt * 64 + (wave & 1) * 32;
-    const int r = l & 31, kq = (l >> 5) * 8;
-    const int am = m0 + r, bn = n0 + r;
-    const bool aValid = am < g.M, bValid = bn < g.N;
-    const int64_t aOff = (int64_t)am * g.a_m, bOff = (int64_t)bn * g.b_n;
-    f32x16 acc = {};
-    const int kBeg = (int)ks * g.kSlice;
-    const int kEnd = (kBeg + g.kSlice < g.K) ? kBeg + g.kSlice : g.K;
-    for (int k0 = kBeg; k0 < kEnd; k0 += 16) {
-        const bf16x8 a = LoadK<AK>(g.A, aValid, aOff, k0 + kq, g.a_k, kEnd);
-        const bf16x8 b = LoadK<BK>(g.B, bValid, bOff, k0 + kq, g.b_k, kEnd);
-        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc, 0, 0, 0);
-    }
-    float* const cf = g.Cf + (int64_t)ks * g.sliceStride;
-    const int n = n0 + r;
-    if (n >= g.N) return;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-        const int m = m0 + (i >> 2) * 8 + (l >> 5) * 4 + (i & 3);
-        if (m >= g.M) continue;
-        const int64_t c = (int64_t)m * g.c_m + (int64_t)n * g.c_n;
-        const float v = acc[i];
-        if (EPI == EPI_F32) {
-            cf[c] = v;
-        } else if (EPI == EPI_BIAS_F32) {
-            g.Cf[c] = v + g.bias[n];
-        } else if (EPI == EPI_BIAS_RELU_BF16) {
-            const float z = v + g.bias[n];
-            g.Cb[c] = hw_f2bf_nonnan(z > 0.0f ? z : 0.0f);
-        } else {
-            const uint16_t mk = g.mask[(int64_t)m * g.mk_m + (int64_t)n * g.mk_n];
-            g.Cb[c] = PositiveBf16(mk) ? hw_f2bf(v) : (uint16_t)0;
-        }
-    }
-}
-
-template <bool AK, bool BK, int EPI>
-static int32_t Gemm(const GemmArgs& g, hipStream_t s)
-{
-    if (g.M <= 0 || g.N <= 0 || g.K <= 0) return Fail(HWPA_ERR_INVALID_ARG, "gemm: empty shape");
-    // Contiguous operands are read 8 elements (16 bytes) at a time.
-    if (AK && (((uintptr_t)g.A & 15) != 0 || (g.a_m & 7) != 0 || g.a_k != 1))
-        return Fail(HWPA_ERR_INVALID_ARG, "gemm: A not 16-byte aligned along k");
-    if (BK && (((uintptr_t)g.B & 15) != 0 || (g.b_n & 7) != 0 || g.b_k != 1))
-        return Fail(HWPA_ERR_INVALID_ARG, "gemm: B not 16-byte aligned along k");
-    GemmArgs h = g;
-    if (h.kSplit <= 1) {
-        h.kSplit = 1;
-        h.kSlice = h.K;
-        h.sliceStride = 0;
-    } else if (EPI != EPI_F32 || h.kSlice % 16 != 0 || (int64_t)h.kSplit * h.kSlice < h.K) {
-        return Fail(HWPA_ERR_INVALID_ARG, "gemm: bad k split");
-    }
-    const uint32_t mt = (uint32_t)((h.M + 63) / 64), nt = (uint32_t)((h.N + 63) / 64);
-    hipLaunchKernelGGL((GemmKernel<AK, BK, EPI>), dim3(mt * nt * (uint32_t)h.kSplit), dim3(256), 0, s, h, nt, mt * nt);
-    return CheckLaunch("GemmKernel");
-}
-
-// out[i] = sum over the kSplit slices of part[ks * n + i], slices in order.
-__global__ __launch_bounds__(256) void SliceSumKernel(const float* __restrict__ part, int32_t slices, int64_t n,
-                                                      float* __restrict__ out)
-{
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= n) return;
-    float acc = 0.0f;
-    for (int32_t k = 0; k < slices; ++k) acc += part[(int64_t)k * n + i];
-    out[i] = acc;
-}
-
-// Weight gradient out[M][N] (row-major) = A^T-like product over a long K
-// (the batch): K is cut into up to kMaxSplit slices of at least 128 rows
-// whose partial products are summed in a fixed order.
-constexpr int kMaxSplit = 32;
-
-template <bool AK, bool BK>
-static int32_t GemmSplitK(GemmArgs g, float* part, float* out, hipStream_t s)
-{
-    int split = (g.K + 127) / 128;
-    split = split < kMaxSplit ? split : kMaxSplit;
-    if (split < 1) split = 1;
-    const int slice = (((g.K + split - 1) / split) + 15) / 16 * 16;
-    split = (g.K + slice - 1) / slice;
-    g.kSplit = split;
-    g.kSlice = slice;
-    g.Cf = part;
-    g.c_m = g.N;
-    g.c_n = 1;
-    g.sliceStride = (int64_t)g.M * g.N;
-    int32_t rc = Gemm<AK, BK, EPI_F32>(g, s);
-    if (rc != HWPA_OK) return rc;
-    const int64_t n = (int64_t)g.M * g.N;
-    hipLaunchKernelGGL(SliceSumKernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, part, split, n, out);
-    return CheckLaunch("SliceSumKernel");
-}
-
-static GemmArgs MakeGemm(int M, int N, int K, const uint16_t* A, int64_t a_m, int64_t a_k, const uint16_t* B,
-                         int64_t b_k, int64_t b_n)
-{
-    GemmArgs g{};
-    g.M = M;
-    g.N = N;
-    g.K = K;
-    g.A = A;
-    g.a_m = a_m;
-    g.a_k = a_k;
-    g.B = B;
-    g.b_k = b_k;
-    g.b_n = b_n;
-    return g;
+    return __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(p));
 }
 
 // ---- features: 300-bin lane histogram -> 128 re-binned, normalised bf16 ----
@@ -249,17 +94,10 @@ __global__ __launch_bounds__(64) void TargetsKernel(const hwpa_lane_hist* __rest
 // + w[7] * BCE(sigmoid(y[11]), r[11]), the last as softplus(y) - r y in its stable form
 // max(y, 0) - r y + log(1 + exp(-|y|)).  Samples marked invalid keep only the last term.
 // omap = {off[6], scale[6], w[8]}.
-__global__ __launch_bounds__(256) void LossKernel(const float* __restrict__ y, const float* __restrict__ t,
-                                                  const uint8_t* __restrict__ valid, uint32_t batch,
-                                                  const float* __restrict__ omap, float* __restrict__ dy,
-                                                  uint16_t* __restrict__ dyb, float* __restrict__ lossPer)
+// One sample: its loss and the gradient g of the batch's mean loss with respect to y.
+__device__ __forceinline__ float SampleLoss(const float* yb, const float* tb, bool valid, float invB, const float* omap,
+                                            float (&g)[MO])
 {
-    const uint32_t b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= batch) return;
-    const float* yb = y + (size_t)b * MO;
-    const float* tb = t + (size_t)b * MO;
-    const float invB = 1.0f / (float)batch;
-    float g[MO];
     // Confidence output: logistic loss against target 11.
     const float wg = omap[19];
     const float yc = yb[11], tc = tb[11];
@@ -267,15 +105,12 @@ __global__ __launch_bounds__(256) void LossKernel(const float* __restrict__ y, c
     float loss = wg * ((hw_maxf(yc, 0.0f) - tc * yc) + hw_logf(1.0f + ez));
     const float sg = (yc >= 0.0f) ? 1.0f / (1.0f + ez) : ez / (1.0f + ez);
     g[11] = (wg * (sg - tc)) * invB;
-    if (valid && valid[b] == 0) {
-        for (int j = 0; j < MO; ++j) {
-            const float gj = (j == 11) ? g[11] : 0.0f;
-            dy[(size_t)b * MO + j] = gj;
-            dyb[(size_t)b * MO + j] = hw_f2bf(gj);
-        }
-        lossPer[b] = loss;
-        return;
+    if (!valid) {
+#pragma unroll
+        for (int j = 0; j < 11; ++j) g[j] = 0.0f;
+        return loss;
     }
+#pragma unroll
     for (int j = 0; j < 6; ++j) {
         const float tn = (tb[j] - omap[j]) / omap[6 + j];
         const float d = yb[j] - tn;
@@ -297,96 +132,385 @@ __global__ __launch_bounds__(256) void LossKernel(const float* __restrict__ y, c
         loss -= wce * (tb[6 + k] * (yb[6 + k] - lse));
         g[6 + k] = (wce * (p - tb[6 + k])) * invB;
     }
-    for (int j = 0; j < MO; ++j) {
-        dy[(size_t)b * MO + j] = g[j];
-        dyb[(size_t)b * MO + j] = hw_f2bf(g[j]);
-    }
-    lossPer[b] = loss;
+    return loss;
 }
 
-// Deterministic mean of per-sample losses (one workgroup, fixed order).
-__global__ __launch_bounds__(256) void MeanKernel(const float* __restrict__ v, uint32_t n, float* __restrict__ out)
+// ---- training ------------------------------------------------------------------
+// A step is two launches: TrainRowsKernel takes every row through the forward pass, the loss and
+// the gradients of its hidden units, TrainGradKernel sums the weight gradients over the batch and
+// takes the Adam step.
+//
+// Between them the matrices lie as the batch-long products read them, [block of 16 rows][unit][16
+// rows], the 16 in the order in which the accumulators of a 32x32 product hold them (the halves
+// of a wave: rows 0-3, 8-11 and 4-7, 12-15): a lane's accumulators are two 16-byte stores, and an
+// operand of a k-step is one contiguous KB.  Any order serves a sum over the batch as long as all
+// matrices share it.
+constexpr int kTrainRows = 32;             // rows of a TrainRowsKernel workgroup
+constexpr int kTrainWaves = MH / 32;       // one wave per 32 hidden units
+constexpr int kGradWaves = 16;
+constexpr int kGradTiles2 = (MH / 32) * (MH / 32), kGradTiles1 = (MH / 32) * (MI / 32), kGradTiles3 = MH / 32;
+constexpr int kGradTiles = kGradTiles2 + kGradTiles1 + kGradTiles3;
+constexpr int kOutPad = 16;                // outputs padded to one k-step
+constexpr int kPart = MO + 1;              // per 32 rows: sums of dY's columns, sum of the losses
+
+// Training buffers, sized for whole 32-row blocks.
+struct TrainActs {
+    uint16_t *X, *H1, *H2, *dH1, *dH2, *dY;
+    float* part;
+};
+
+struct AdamArgs {
+    float *P, *Mo, *Ve;
+    uint16_t *Pb, *WT;
+    float lr, b1, b2, c1, c2, eps;
+};
+
+// bf16 mirrors of the weights in operand order, [16-wide k-step][unit][16 k], so that a wave reads a
+// k-step of 32 units as one KB: W1, W2, and transposed W2 and W3 (its k-step padded with zeros).
+constexpr size_t OFF_O1 = 0;
+constexpr size_t OFF_O2 = OFF_O1 + (size_t)MH * MI;
+constexpr size_t OFF_T2 = OFF_O2 + (size_t)MH * MH;
+constexpr size_t OFF_T3 = OFF_T2 + (size_t)MH * MH;
+constexpr size_t NTRANS = OFF_T3 + (size_t)MH * kOutPad;
+
+__device__ __forceinline__ uint32_t OperandAt(uint32_t unit, uint32_t k) { return ((k >> 4) * MH + unit) * 16 + (k & 15); }
+
+// Parameter i into the bf16 mirrors.
+__device__ __forceinline__ void StoreBf16(uint32_t i, float v, uint16_t* __restrict__ pb, uint16_t* __restrict__ wt)
 {
-    __shared__ float part[256];
-    float s = 0.0f;
-    for (uint32_t i = threadIdx.x; i < n; i += 256) s += v[i];
-    part[threadIdx.x] = s;
+    const uint16_t h = hw_f2bf(v);
+    pb[i] = h;
+    if (i < OFF_B1) {
+        wt[OFF_O1 + OperandAt(i / MI, i % MI)] = h;
+    } else if (i >= OFF_W2 && i < OFF_B2) {
+        const uint32_t e = i - (uint32_t)OFF_W2;
+        wt[OFF_O2 + OperandAt(e / MH, e % MH)] = h;
+        wt[OFF_T2 + OperandAt(e % MH, e / MH)] = h;
+    } else if (i >= OFF_W3 && i < OFF_B3) {
+        const uint32_t e = i - (uint32_t)OFF_W3;
+        wt[OFF_T3 + OperandAt(e % MH, e / MH)] = h;
+    }
+}
+
+__global__ __launch_bounds__(256) void ToBf16Kernel(const float* __restrict__ p, uint16_t* __restrict__ pb,
+                                                    uint16_t* __restrict__ wt, uint32_t n)
+{
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) StoreBf16(i, p[i], pb, wt);
+    if (i < MH * (kOutPad - MO)) wt[OFF_T3 + (size_t)(i / (kOutPad - MO)) * kOutPad + MO + i % (kOutPad - MO)] = 0;
+}
+
+// Forward, loss and hidden gradients of 32 rows per workgroup, one wave per 32 hidden units.  At a
+// training batch the kernel is a chain of small products, so what bounds it is latency: every wave
+// requests its share of the weights well before their products (8 + 16 + 16 k-steps, 40 KB, one
+// contiguous KB each: read in the parameters' own order, 32 B of each line at a time, the kernel
+// took 30 us), targets and output weights are staged with the inputs, the activations go from
+// layer to layer in LDS, and the ReLU masks stay in registers.  Batch 4,096 (128 workgroups): 17
+// us, where the forward pass (16 workgroups of 256 rows), the loss and two products with operands
+// gathered 2 bytes at a time took 36 + 5 + 11 + 20 us.
+__global__ __launch_bounds__(64 * kTrainWaves) void TrainRowsKernel(const uint16_t* __restrict__ x,
+                                                                    const float* __restrict__ t,
+                                                                    const uint8_t* __restrict__ valid, uint32_t batch,
+                                                                    const uint16_t* __restrict__ Wb,
+                                                                    const uint16_t* __restrict__ WT,
+                                                                    const float* __restrict__ P,
+                                                                    const float* __restrict__ omap, TrainActs w)
+{
+    constexpr int kXs = MI + 8, kHs = MH + 8, kYs = 24;
+    __shared__ __align__(16) uint16_t xs[kTrainRows][kXs];
+    __shared__ __align__(16) uint16_t hs[3][kTrainRows][kHs];   // h1, h2, dh2
+    __shared__ __align__(16) uint16_t dys[kTrainRows][kYs];
+    __shared__ __align__(16) uint16_t w3s[MO][kHs];
+    __shared__ float ys[kTrainRows][MO + 1], dyf[kTrainRows][kPart], ts[kTrainRows][MO + 1], om[20];
+    __shared__ uint8_t vs[kTrainRows];
+    static_assert(64 * kTrainWaves == kTrainRows * MI / 8, "one 16-byte piece of the inputs per thread");
+    const int wave = threadIdx.x >> 6, l = threadIdx.x & 63, r = l & 31, half = l >> 5, kq = half * 8;
+    const int n = wave * 32 + r;   // this lane's hidden unit
+    bf16x8 w1[MI / 16], w2[MH / 16], wt[MH / 16];
+#pragma unroll
+    for (int k = 0; k < MI / 16; ++k) w1[k] = LoadRow8(WT + OFF_O1 + ((size_t)k * MH + n) * 16 + kq);
+#pragma unroll
+    for (int k = 0; k < MH / 16; ++k) w2[k] = LoadRow8(WT + OFF_O2 + ((size_t)k * MH + n) * 16 + kq);
+    const bf16x8 w3t = LoadRow8(WT + OFF_T3 + (size_t)n * kOutPad + kq);
+    const float b1 = P[OFF_B1 + n], b2 = P[OFF_B2 + n], b3 = P[OFF_B3 + (r < MO ? r : 0)];
+    const float invB = 1.0f / (float)batch;
+    auto rowOf = [&](int i) { return (i >> 2) * 8 + half * 4 + (i & 3); };
+    auto pack = [](uint32_t lo, uint32_t hi) { return lo | (hi << 16); };
+    const uint32_t blk = blockIdx.x;
+    const uint32_t m0 = blk * kTrainRows;
+    const uint32_t live = min(batch - m0, (uint32_t)kTrainRows);
+    // A lane's 16 values of one unit: two pieces of the batch-long layout.
+    auto storeUnits = [&](uint16_t* base, const uint32_t (&v)[8]) {
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
+            *reinterpret_cast<uint4*>(base + ((((size_t)blk * 2 + q) * MH + n) * 2 + half) * 8) =
+                make_uint4(v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]);
+    };
+    auto storeRows = [&](uint16_t (*h)[kHs], const uint32_t (&v)[8]) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            h[rowOf(2 * i)][n] = (uint16_t)v[i];
+            h[rowOf(2 * i + 1)][n] = (uint16_t)(v[i] >> 16);
+        }
+    };
+    // Rows past the batch are zero throughout.
+    {
+        const int row = threadIdx.x >> 4, c = (threadIdx.x & 15) * 8;
+        uint4 v = make_uint4(0u, 0u, 0u, 0u);
+        if ((uint32_t)row < live) v = *reinterpret_cast<const uint4*>(x + (size_t)(m0 + row) * MI + c);
+        float tv = 0.0f;
+        uint4 wv = make_uint4(0u, 0u, 0u, 0u);
+        static_assert(kTrainRows * MO <= 64 * kTrainWaves && MO * MH / 8 <= 64 * kTrainWaves, "one load per thread");
+        if (threadIdx.x < live * MO) tv = t[(size_t)m0 * MO + threadIdx.x];
+        if (threadIdx.x < MO * MH / 8) wv = *reinterpret_cast<const uint4*>(Wb + OFF_W3 + (size_t)threadIdx.x * 8);
+        if (threadIdx.x < 20) om[threadIdx.x] = omap[threadIdx.x];
+        if (threadIdx.x < live) vs[threadIdx.x] = !valid || valid[m0 + threadIdx.x] != 0;
+        *reinterpret_cast<uint4*>(&xs[row][c]) = v;
+        if (threadIdx.x < kTrainRows * MO) ts[threadIdx.x / MO][threadIdx.x % MO] = tv;
+        if (threadIdx.x < MO * MH / 8)
+            *reinterpret_cast<uint4*>(&w3s[threadIdx.x / (MH / 8)][threadIdx.x % (MH / 8) * 8]) = wv;
+    }
     __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w) part[threadIdx.x] += part[threadIdx.x + w];
-        __syncthreads();
+    {
+        const int q = threadIdx.x >> 8, f = (threadIdx.x >> 1) & (MI - 1), hf = threadIdx.x & 1;
+        uint32_t v[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int row = q * 16 + (j >> 1) * 8 + hf * 4 + (j & 1) * 2;
+            v[j] = pack(xs[row][f], xs[row + 1][f]);
+        }
+        *reinterpret_cast<uint4*>(w.X + ((((size_t)blk * 2 + q) * MI + f) * 2 + hf) * 8) =
+            make_uint4(v[0], v[1], v[2], v[3]);
     }
-    if (threadIdx.x == 0) *out = part[0] / (float)n;
-}
-
-// Column sums of a [rows][cols] matrix (bf16 or fp32), two fixed-order passes.
-// Rows per partial sum of the bias-gradient column sums: batch / 32 workgroups, each
-// thread with its 32 loads in flight; the partials are then added in slice order.
-constexpr int COLSUM_ROWS = 32;
-template <typename T>
-__device__ __forceinline__ float LoadVal(const T* p, size_t i);
-template <>
-__device__ __forceinline__ float LoadVal<float>(const float* p, size_t i) { return p[i]; }
-template <>
-__device__ __forceinline__ float LoadVal<uint16_t>(const uint16_t* p, size_t i) { return hw_bf2f(p[i]); }
-
-template <typename T>
-__global__ __launch_bounds__(256) void ColSumPartKernel(const T* __restrict__ d, uint32_t rows, uint32_t cols,
-                                                        float* __restrict__ part)
-{
-    const uint32_t c = threadIdx.x + blockIdx.y * 256;
-    if (c >= cols) return;
-    const uint32_t r0 = blockIdx.x * COLSUM_ROWS;
-    const uint32_t r1 = min(rows, r0 + COLSUM_ROWS);
-    // All loads of the slice are issued before the (row-ordered) adds.
-    float v[COLSUM_ROWS];
+    f32x16 acc{};
 #pragma unroll
-    for (int i = 0; i < COLSUM_ROWS; ++i) v[i] = (r0 + i < r1) ? LoadVal<T>(d, (size_t)(r0 + i) * cols + c) : 0.0f;
-    float s = 0.0f;
+    for (int k = 0; k < MI / 16; ++k)
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(LoadRow8(&xs[r][16 * k + kq]), w1[k], acc, 0, 0, 0);
+    auto relu = [&](float b, uint32_t (&v)[8]) {
 #pragma unroll
-    for (int i = 0; i < COLSUM_ROWS; ++i) s += v[i];
-    part[(size_t)blockIdx.x * cols + c] = s;
-}
-
-__global__ __launch_bounds__(256) void ColSumFinalKernel(const float* __restrict__ part, uint32_t chunks,
-                                                         uint32_t cols, float* __restrict__ out)
-{
-    const uint32_t c = blockIdx.x * 256 + threadIdx.x;
-    if (c >= cols) return;
-    // Partials in slice order, 16 loads in flight at a time.
-    float s = 0.0f;
-    for (uint32_t k0 = 0; k0 < chunks; k0 += 16) {
-        float v[16];
+        for (int i = 0; i < 16; ++i) {
+            const float z = acc[i] + b;
+            uint32_t h = hw_f2bf_nonnan(z > 0.0f ? z : 0.0f);
+            if ((uint32_t)rowOf(i) >= live) h = 0;
+            v[i >> 1] = (i & 1) ? pack(v[i >> 1], h) : h;
+        }
+    };
+    auto masked = [&](const uint32_t (&h)[8], uint32_t (&v)[8]) {
 #pragma unroll
-        for (int i = 0; i < 16; ++i) v[i] = (k0 + i < chunks) ? part[(size_t)(k0 + i) * cols + c] : 0.0f;
+        for (int i = 0; i < 16; ++i) {
+            const uint32_t d =
+                PositiveBf16((uint16_t)(h[i >> 1] >> (16 * (i & 1)))) ? (uint32_t)hw_f2bf(acc[i]) : 0u;
+            v[i >> 1] = (i & 1) ? pack(v[i >> 1], d) : d;
+        }
+    };
 #pragma unroll
-        for (int i = 0; i < 16; ++i) s += v[i];
+    for (int k = 0; k < MH / 16; ++k) wt[k] = LoadRow8(WT + OFF_T2 + ((size_t)k * MH + n) * 16 + kq);
+    uint32_t h1[8], h2[8], d[8];
+    relu(b1, h1);
+    storeRows(hs[0], h1);
+    storeUnits(w.H1, h1);
+    __syncthreads();
+    acc = f32x16{};
+#pragma unroll
+    for (int k = 0; k < MH / 16; ++k)
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(LoadRow8(&hs[0][r][16 * k + kq]), w2[k], acc, 0, 0, 0);
+    relu(b2, h2);
+    storeRows(hs[1], h2);
+    storeUnits(w.H2, h2);
+    __syncthreads();
+    if (wave == 0) {
+        // Outputs: one 32-column product of which MO columns are real.
+        const bf16x8 zero8 = __builtin_bit_cast(bf16x8, make_uint4(0u, 0u, 0u, 0u));
+        acc = f32x16{};
+#pragma unroll
+        for (int k = 0; k < MH / 16; ++k) {
+            const bf16x8 w3 = r < MO ? LoadRow8(&w3s[r][16 * k + kq]) : zero8;
+            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(LoadRow8(&hs[1][r][16 * k + kq]), w3, acc, 0, 0, 0);
+        }
+        if (r < MO) {
+#pragma unroll
+            for (int i = 0; i < 16; ++i) ys[rowOf(i)][r] = acc[i] + b3;
+        }
     }
-    out[c] = s;
+    __syncthreads();
+    if (threadIdx.x < (unsigned)kTrainRows) {
+        float g[MO] = {}, loss = 0.0f;
+        if (threadIdx.x < live) {
+            loss = SampleLoss(ys[threadIdx.x], ts[threadIdx.x], vs[threadIdx.x] != 0, invB, om, g);
+        }
+#pragma unroll
+        for (int j = 0; j < kOutPad; ++j) dys[threadIdx.x][j] = j < MO ? hw_f2bf(g[j < MO ? j : 0]) : (uint16_t)0;
+#pragma unroll
+        for (int j = 0; j < MO; ++j) dyf[threadIdx.x][j] = g[j];
+        dyf[threadIdx.x][MO] = loss;
+    }
+    __syncthreads();
+    if (threadIdx.x < kPart) {
+        float s = 0.0f;
+#pragma unroll
+        for (int i = 0; i < kTrainRows; ++i) s += dyf[i][threadIdx.x];
+        w.part[(size_t)blk * kPart + threadIdx.x] = s;
+    } else if (wave == 1) {
+        const int q = l >> 5, o = (l >> 1) & (kOutPad - 1), hf = l & 1;
+        uint32_t v[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int row = q * 16 + (j >> 1) * 8 + hf * 4 + (j & 1) * 2;
+            v[j] = pack(dys[row][o], dys[row + 1][o]);
+        }
+        *reinterpret_cast<uint4*>(w.dY + ((((size_t)blk * 2 + q) * kOutPad + o) * 2 + hf) * 8) =
+            make_uint4(v[0], v[1], v[2], v[3]);
+    }
+    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(LoadRow8(&dys[r][kq]), w3t, f32x16{}, 0, 0, 0);
+    masked(h2, d);
+    storeRows(hs[2], d);
+    storeUnits(w.dH2, d);
+    __syncthreads();
+    acc = f32x16{};
+#pragma unroll
+    for (int k = 0; k < MH / 16; ++k)
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(LoadRow8(&hs[2][r][16 * k + kq]), wt[k], acc, 0, 0, 0);
+    masked(h1, d);
+    storeUnits(w.dH1, d);
 }
 
-__global__ __launch_bounds__(256) void AdamKernel(float* __restrict__ p, const float* __restrict__ g,
-                                                  float* __restrict__ m, float* __restrict__ v,
-                                                  uint16_t* __restrict__ pb, uint32_t n, float lr, float b1,
-                                                  float b2, float c1, float c2, float eps)
+__device__ __forceinline__ void AdamOne(uint32_t i, float gi, float p0, float m0, float v0, const AdamArgs& a)
 {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const float gi = g[i];
-    const float mi = b1 * m[i] + (1.0f - b1) * gi;
-    const float vi = b2 * v[i] + (1.0f - b2) * (gi * gi);
-    m[i] = mi;
-    v[i] = vi;
-    const float mh = mi / c1, vh = vi / c2;
-    const float pi = p[i] - lr * mh / (hw_sqrtf(vh) + eps);
-    p[i] = pi;
-    pb[i] = hw_f2bf(pi);
+    const float mi = a.b1 * m0 + (1.0f - a.b1) * gi;
+    const float vi = a.b2 * v0 + (1.0f - a.b2) * (gi * gi);
+    a.Mo[i] = mi;
+    a.Ve[i] = vi;
+    const float mh = mi / a.c1, vh = vi / a.c2;
+    const float pi = p0 - a.lr * mh / (hw_sqrtf(vh) + a.eps);
+    a.P[i] = pi;
+    StoreBf16(i, pi, a.Pb, a.WT);
 }
 
-__global__ __launch_bounds__(256) void ToBf16Kernel(const float* __restrict__ p, uint16_t* __restrict__ pb, uint32_t n)
+// Weight gradients: one workgroup per 32x32 tile of W1, W2 and W3, its 16 waves taking every 16th
+// 16-row block of the batch, their accumulators added in wave order through LDS; the bias gradients of
+// W1 and W2 are one more product, with ones, of the tiles in the first column; the last workgroup
+// adds the per-block sums of the outputs' gradients and of the losses.  STEP applies the Adam
+// step to the sums, else they go to G.  Bound by the operand reads: 512 KB a tile at batch 4,096,
+// contiguous, from the L2s (consecutive workgroups, which lie on different XCDs, differ in the
+// tile's rows, so an XCD reads one eighth of one operand).  9 us there (10 with the step); split over
+// the batch into 32 slices with operands gathered 2 bytes at a time, the three products took 65 us,
+// the sums of the slices 27, of the columns 36 and of the losses 6, the Adam step 4.
+template <bool STEP>
+__global__ __launch_bounds__(64 * kGradWaves) void TrainGradKernel(TrainActs w, uint32_t batch, float* __restrict__ G,
+                                                                   float* __restrict__ lossOut, AdamArgs a)
 {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) pb[i] = hw_f2bf(p[i]);
+    __shared__ float red[kGradWaves][32 * 32];
+    __shared__ float redB[kGradWaves][32];
+    const int wave = threadIdx.x >> 6, l = threadIdx.x & 63, r = l & 31, half = l >> 5;
+    const uint32_t blocks = (batch + kTrainRows - 1) / kTrainRows;
+    auto emit = [&](uint32_t i, float g, float p0, float m0, float v0) {
+        if (STEP) AdamOne(i, g, p0, m0, v0, a);
+        else G[i] = g;
+    };
+    int tile = (int)blockIdx.x;
+    if (tile == kGradTiles) {
+        static_assert(kPart <= kGradWaves, "one wave per sum");
+        if (wave >= kPart) return;
+        float s = 0.0f;
+        for (uint32_t b = (uint32_t)l; b < blocks; b += 64) s += w.part[(size_t)b * kPart + wave];
+        for (int m = 32; m > 0; m >>= 1) s += __shfl_xor(s, m, 64);
+        if (l != 0) return;
+        if (wave == MO) {
+            *lossOut = s / (float)batch;
+        } else {
+            const uint32_t i = (uint32_t)OFF_B3 + (uint32_t)wave;
+            if (STEP) emit(i, s, a.P[i], a.Mo[i], a.Ve[i]);
+            else emit(i, s, 0.0f, 0.0f, 0.0f);
+        }
+        return;
+    }
+    const uint16_t *A, *B;
+    int nfA = MH, nfB = MH, rows = 32, m0, n0;
+    uint32_t off, offB = 0;
+    bool bias = false;
+    if (tile < kGradTiles2) {
+        m0 = (tile % (MH / 32)) * 32;
+        n0 = (tile / (MH / 32)) * 32;
+        A = w.dH2;
+        B = w.H1;
+        off = (uint32_t)OFF_W2;
+        offB = (uint32_t)OFF_B2;
+        bias = n0 == 0;
+    } else if (tile < kGradTiles2 + kGradTiles1) {
+        tile -= kGradTiles2;
+        m0 = (tile % (MH / 32)) * 32;
+        n0 = (tile / (MH / 32)) * 32;
+        A = w.dH1;
+        B = w.X;
+        nfB = MI;
+        off = (uint32_t)OFF_W1;
+        offB = (uint32_t)OFF_B1;
+        bias = n0 == 0;
+    } else {
+        m0 = 0;
+        n0 = (tile - kGradTiles2 - kGradTiles1) * 32;
+        A = w.dY;
+        B = w.H2;
+        nfA = kOutPad;
+        rows = MO;
+        off = (uint32_t)OFF_W3;
+    }
+    // This thread's element of the tile, and its parameter's state in flight meanwhile.
+    const int em = (wave >> 2) * 8 + half * 4 + (wave & 3), en = r;
+    const uint32_t ei = off + (uint32_t)(m0 + em) * (uint32_t)nfB + (uint32_t)(n0 + en);
+    const uint32_t bi = offB + (uint32_t)m0 + (uint32_t)r;
+    const bool mine = em < rows, mineB = bias && threadIdx.x < 32;
+    float p0 = 0.0f, mo = 0.0f, ve = 0.0f, pB = 0.0f, moB = 0.0f, veB = 0.0f;
+    if (STEP && mine) {
+        p0 = a.P[ei];
+        mo = a.Mo[ei];
+        ve = a.Ve[ei];
+    }
+    if (STEP && mineB) {
+        pB = a.P[bi];
+        moB = a.Mo[bi];
+        veB = a.Ve[bi];
+    }
+    const bf16x8 zero8 = __builtin_bit_cast(bf16x8, make_uint4(0u, 0u, 0u, 0u));
+    const bf16x8 ones = __builtin_bit_cast(bf16x8, make_uint4(0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u));
+    const uint32_t kb = blocks * 2;
+    const bool aRow = r < nfA;
+    const uint16_t* pa = A + ((size_t)(m0 + (aRow ? r : 0)) * 2 + half) * 8;
+    const uint16_t* pb = B + ((size_t)(n0 + r) * 2 + half) * 8;
+    const size_t sa = (size_t)nfA * 16, sb = (size_t)nfB * 16;
+    f32x16 acc{}, accB{};
+    constexpr uint32_t kDeep = 4;
+    for (uint32_t k0 = (uint32_t)wave; k0 < kb; k0 += kGradWaves * kDeep) {
+        bf16x8 va[kDeep], vb[kDeep];
+#pragma unroll
+        for (uint32_t j = 0; j < kDeep; ++j) {
+            const uint32_t k = k0 + j * kGradWaves;
+            va[j] = (aRow && k < kb) ? LoadRow8(pa + sa * k) : zero8;
+            vb[j] = k < kb ? LoadRow8(pb + sb * k) : zero8;
+        }
+#pragma unroll
+        for (uint32_t j = 0; j < kDeep; ++j) {
+            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va[j], vb[j], acc, 0, 0, 0);
+            if (bias) accB = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va[j], ones, accB, 0, 0, 0);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < 16; ++i) red[wave][i * 64 + l] = acc[i];
+    if (bias && r == 0) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) redB[wave][(i >> 2) * 8 + half * 4 + (i & 3)] = accB[i];
+    }
+    __syncthreads();
+    float g = 0.0f;
+#pragma unroll
+    for (int k = 0; k < kGradWaves; ++k) g += red[k][threadIdx.x];
+    if (mine) emit(ei, g, p0, mo, ve);
+    if (mineB) {
+        float gb = 0.0f;
+#pragma unroll
+        for (int k = 0; k < kGradWaves; ++k) gb += redB[k][r];
+        emit(bi, gb, pB, moB, veB);
+    }
 }
 
 }  // namespace hwpa
@@ -400,23 +524,12 @@ struct hwpa_initializer {
     float* Mo = nullptr;    // Adam moments
     float* Ve = nullptr;
     int64_t step = 0;
-    // activations, sized for `rows`
-    uint32_t rows = 0;
-    uint16_t* H1 = nullptr;
-    uint16_t* H2 = nullptr;
-    float* Y = nullptr;
-    // training buffers, sized for `batchCap`
-    uint32_t batchCap = 0;
-    float* dY = nullptr;
-    uint16_t* dYb = nullptr;
-    uint16_t* dH1 = nullptr;
-    uint16_t* dH2 = nullptr;
-    float* lossPer = nullptr;
-    float* colPart = nullptr;
+    uint16_t* WT = nullptr; // transposed bf16 mirrors (NTRANS)
+    uint32_t batchCap = 0;  // rows the training buffers hold, whole 32-row blocks
+    TrainActs acts{};
     float* lossDev = nullptr;
     float* omap = nullptr;      // device {off[6], scale[6], w[8]}
     float omapHost[20] = {};
-    float* kPart = nullptr;     // split-K partial weight gradients, kMaxSplit x MH x MH
     // A learned-start workspace kept between estimations (LearnedWsTake), at most one.
     std::mutex wsMutex;
     LearnedWs ws;
@@ -452,98 +565,51 @@ void LearnedWsGive(hwpa_initializer* m, LearnedWs& w)
     LearnedWsFree(w);
 }
 
-static void FreeActs(hwpa_initializer* m)
-{
-    DeviceFree(m->H1);
-    DeviceFree(m->H2);
-    DeviceFree(m->Y);
-    m->H1 = m->H2 = nullptr;
-    m->Y = nullptr;
-    m->rows = 0;
-}
-
 static void FreeTrain(hwpa_initializer* m)
 {
-    DeviceFree(m->dY);
-    DeviceFree(m->dYb);
-    DeviceFree(m->dH1);
-    DeviceFree(m->dH2);
-    DeviceFree(m->lossPer);
-    DeviceFree(m->colPart);
-    m->dY = nullptr;
-    m->dYb = m->dH1 = m->dH2 = nullptr;
-    m->lossPer = m->colPart = nullptr;
+    DeviceFree(m->acts.X);
+    DeviceFree(m->acts.H1);
+    DeviceFree(m->acts.H2);
+    DeviceFree(m->acts.dH1);
+    DeviceFree(m->acts.dH2);
+    DeviceFree(m->acts.dY);
+    DeviceFree(m->acts.part);
+    m->acts = TrainActs{};
     m->batchCap = 0;
-}
-
-static int32_t EnsureRows(hwpa_initializer* m, uint32_t rows)
-{
-    if (rows <= m->rows) return HWPA_OK;
-    // Buffers may still be in use by queued work on any stream.
-    HWPA_HIP(hipDeviceSynchronize());
-    FreeActs(m);
-    int32_t rc = DeviceAlloc((void**)&m->H1, (size_t)rows * MH * 2, "mlp activations");
-    if (rc == HWPA_OK) rc = DeviceAlloc((void**)&m->H2, (size_t)rows * MH * 2, "mlp activations");
-    if (rc == HWPA_OK) rc = DeviceAlloc((void**)&m->Y, (size_t)rows * MO * 4, "mlp outputs");
-    if (rc != HWPA_OK) {
-        FreeActs(m);
-        return rc;
-    }
-    m->rows = rows;
-    return HWPA_OK;
 }
 
 static int32_t EnsureBatch(hwpa_initializer* m, uint32_t batch)
 {
-    int32_t rc = EnsureRows(m, batch);
-    if (rc != HWPA_OK || batch <= m->batchCap) return rc;
+    if (batch <= m->batchCap) return HWPA_OK;
+    // Buffers may still be in use by queued work on any stream.
     HWPA_HIP(hipDeviceSynchronize());
     FreeTrain(m);
-    const size_t chunks = (batch + COLSUM_ROWS - 1) / COLSUM_ROWS;
-    rc = DeviceAlloc((void**)&m->dY, (size_t)batch * MO * 4, "mlp gradients");
-    if (rc == HWPA_OK) rc = DeviceAlloc((void**)&m->dYb, (size_t)batch * MO * 2, "mlp gradients");
-    if (rc == HWPA_OK) rc = DeviceAlloc((void**)&m->dH1, (size_t)batch * MH * 2, "mlp gradients");
-    if (rc == HWPA_OK) rc = DeviceAlloc((void**)&m->dH2, (size_t)batch * MH * 2, "mlp gradients");
-    if (rc == HWPA_OK) rc = DeviceAlloc((void**)&m->lossPer, (size_t)batch * 4, "mlp loss");
-    if (rc == HWPA_OK) rc = DeviceAlloc((void**)&m->colPart, chunks * MH * 4, "mlp bias sums");
+    const size_t blocks = ((size_t)batch + kTrainRows - 1) / kTrainRows, rows = blocks * kTrainRows;
+    TrainActs& w = m->acts;
+    int32_t rc = DeviceAlloc((void**)&w.X, rows * MI * 2, "mlp activations");
+    if (rc == HWPA_OK) rc = DeviceAlloc((void**)&w.H1, rows * MH * 2, "mlp activations");
+    if (rc == HWPA_OK) rc = DeviceAlloc((void**)&w.H2, rows * MH * 2, "mlp activations");
+    if (rc == HWPA_OK) rc = DeviceAlloc((void**)&w.dH1, rows * MH * 2, "mlp gradients");
+    if (rc == HWPA_OK) rc = DeviceAlloc((void**)&w.dH2, rows * MH * 2, "mlp gradients");
+    if (rc == HWPA_OK) rc = DeviceAlloc((void**)&w.dY, rows * kOutPad * 2, "mlp gradients");
+    if (rc == HWPA_OK) rc = DeviceAlloc((void**)&w.part, blocks * kPart * 4, "mlp bias sums");
     if (rc != HWPA_OK) {
         FreeTrain(m);
         return rc;
     }
-    m->batchCap = batch;
+    m->batchCap = (uint32_t)std::min<size_t>(rows, UINT32_MAX);
     return HWPA_OK;
 }
 
-static int32_t ColSum(const void* d, bool bf16, uint32_t rows, uint32_t cols, float* part, float* out, hipStream_t s)
-{
-    const uint32_t chunks = (rows + COLSUM_ROWS - 1) / COLSUM_ROWS;
-    const dim3 grid(chunks, (cols + 255) / 256);
-    if (bf16)
-        hipLaunchKernelGGL(ColSumPartKernel<uint16_t>, grid, dim3(256), 0, s, (const uint16_t*)d, rows, cols, part);
-    else
-        hipLaunchKernelGGL(ColSumPartKernel<float>, grid, dim3(256), 0, s, (const float*)d, rows, cols, part);
-    int32_t rc = CheckLaunch("ColSumPartKernel");
-    if (rc != HWPA_OK) return rc;
-    hipLaunchKernelGGL(ColSumFinalKernel, dim3((cols + 255) / 256), dim3(256), 0, s, part, chunks, cols, out);
-    return CheckLaunch("ColSumFinalKernel");
-}
-
-// Fused forward pass: 32 rows per wave, kFusedWaves (8) waves per workgroup.  Each layer is the
-// 32x32x16 bf16 MFMA over 32-column tiles with k ascending -- the arithmetic of
-// GemmKernel, so outputs equal the three-GEMM pass bit for bit -- but the hidden
-// activations stay in LDS (row-major, read back as the next layer's operand) instead of
-// HBM; h1 / h2 are written out only when given (training keeps them for the backward
-// pass).  The weights of each 16-wide k-step of layers 1 and 2 (all 256 output columns:
+// Inference: 32 rows per wave, kFusedWaves (8) waves per workgroup.  Each layer is the
+// 32x32x16 bf16 MFMA over 32-column tiles with k ascending, the arithmetic of the training
+// kernels' forward pass; the hidden activations stay in LDS (row-major, read back as the next
+// layer's operand).  The weights of each 16-wide k-step of layers 1 and 2 (all 256 output columns:
 // 8 KB) are staged once per workgroup in LDS, double-buffered with one barrier per step, so
 // the 8 waves (256 rows) of a workgroup share one read of them instead of each wave
 // fetching all 192 KB from L2.
 constexpr int kFusedRows = 32, kFusedWaves = 8, kHsStride = MH + 8;
 constexpr int kSlab = MH * 16;   // bf16 weights of one k-step: [256 columns][16 k]
-
-__device__ __forceinline__ bf16x8 LoadRow8(const uint16_t* __restrict__ p)
-{
-    return __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(p));
-}
 
 // HIST: the inputs are computed from the lane histograms as FeaturesKernel does (row =
 // lane * 64 + ZMW), so inference reads the counters once and writes no input matrix.  Each
@@ -554,8 +620,7 @@ template <bool HIST>
 __global__ __launch_bounds__(64 * kFusedWaves) void MlpFusedForwardKernel(const uint16_t* __restrict__ x,
                                                              const hwpa_lane_hist* __restrict__ hists, uint32_t rows,
                                                              const uint16_t* __restrict__ Wb,
-                                                             const float* __restrict__ P, float* __restrict__ y,
-                                                             uint16_t* __restrict__ h1out, uint16_t* __restrict__ h2out)
+                                                             const float* __restrict__ P, float* __restrict__ y)
 {
     __shared__ __align__(16) uint16_t hs[kFusedWaves][kFusedRows][kHsStride];
     __shared__ __align__(16) uint16_t ws[2][kSlab];
@@ -581,9 +646,9 @@ __global__ __launch_bounds__(64 * kFusedWaves) void MlpFusedForwardKernel(const 
     // the tile (f32x16 layout of the 32x32 MFMA) for row r: each lane holds four runs of four
     // consecutive features of its own row.
     auto outRow = [&](int i) { return (i >> 2) * 8 + (l >> 5) * 4 + (i & 3); };
-    // Bias, ReLU, bf16 and the row's activations back into LDS (and to hout when given): one
-    // 8-byte store per run of four features.
-    auto hiddenOut = [&](const f32x16 (&a)[MH / 32], int boff, uint16_t* hout) {
+    // Bias, ReLU, bf16 and the row's activations back into LDS: one 8-byte store per run of four
+    // features.
+    auto hiddenOut = [&](const f32x16 (&a)[MH / 32], int boff) {
 #pragma unroll
         for (int j = 0; j < MH / 32; ++j) {
 #pragma unroll
@@ -599,7 +664,6 @@ __global__ __launch_bounds__(64 * kFusedWaves) void MlpFusedForwardKernel(const 
                 }
                 const uint2 pk = make_uint2(hv[0] | (hv[1] << 16), hv[2] | (hv[3] << 16));
                 *reinterpret_cast<uint2*>(hp(r, f0)) = pk;
-                if (hout && rowValid) *reinterpret_cast<uint2*>(hout + (m0 + r) * MH + f0) = pk;
             }
         }
     };
@@ -678,7 +742,7 @@ __global__ __launch_bounds__(64 * kFusedWaves) void MlpFusedForwardKernel(const 
         next = next2;
         __syncthreads();
     }
-    hiddenOut(acc, OFF_B1, h1out);
+    hiddenOut(acc, OFF_B1);
     __syncthreads();
 
     // ---- layer 2: [32 x MH] x [MH x MH]
@@ -703,7 +767,7 @@ __global__ __launch_bounds__(64 * kFusedWaves) void MlpFusedForwardKernel(const 
         next = next2;
         __syncthreads();
     }
-    hiddenOut(acc, OFF_B2, h2out);
+    hiddenOut(acc, OFF_B2);
     __syncthreads();
 
     // ---- layer 3: [32 x MH] x [MH x MO], one 32-column tile of which MO columns are real
@@ -725,16 +789,15 @@ __global__ __launch_bounds__(64 * kFusedWaves) void MlpFusedForwardKernel(const 
     }
 }
 
-// Forward pass over `rows` inputs through the activation buffers h1, h2 into y.
-static int32_t Forward(const hwpa_initializer* m, const uint16_t* x, uint32_t rows, float* y, uint16_t* h1,
-                       uint16_t* h2, hipStream_t s)
+// Forward pass over `rows` inputs into y.
+static int32_t Forward(const hwpa_initializer* m, const uint16_t* x, uint32_t rows, float* y, hipStream_t s)
 {
     if (rows == 0) return Fail(HWPA_ERR_INVALID_ARG, "mlp forward: no rows");
     if (((uintptr_t)x & 15) != 0) return Fail(HWPA_ERR_INVALID_ARG, "mlp forward: input not 16-byte aligned");
     const uint32_t per = (uint32_t)(kFusedRows * kFusedWaves);
     hipLaunchKernelGGL(MlpFusedForwardKernel<false>, dim3((rows + per - 1) / per), dim3(64 * kFusedWaves), 0, s, x,
                        nullptr, rows,
-                       m->Pb, m->P, y, h1, h2);
+                       m->Pb, m->P, y);
     return CheckLaunch("MlpFusedForwardKernel");
 }
 
@@ -750,53 +813,25 @@ static int32_t ForwardFromHist(const hwpa_initializer* m, const hwpa_lane_hist* 
     const uint32_t per = (uint32_t)(kFusedRows * kFusedWaves);
     hipLaunchKernelGGL(MlpFusedForwardKernel<true>, dim3((rows + per - 1) / per), dim3(64 * kFusedWaves), 0, s, nullptr,
                        hist, rows,
-                       m->Pb, m->P, y, nullptr, nullptr);
+                       m->Pb, m->P, y);
     return CheckLaunch("MlpFusedForwardKernel");
 }
 
-// Loss and gradients of the mean loss over a batch; gradients into m->G.
+// Mean loss of a batch into m->lossDev; its gradients into m->G, or (step given) applied.
 static int32_t Backward(hwpa_initializer* m, const uint16_t* x, const float* t, const uint8_t* valid, uint32_t batch,
-                        hipStream_t s)
+                        const AdamArgs* step, hipStream_t s)
 {
-    int32_t rc = Forward(m, x, batch, m->Y, m->H1, m->H2, s);
+    const uint32_t blocks = (uint32_t)(((uint64_t)batch + kTrainRows - 1) / kTrainRows);
+    hipLaunchKernelGGL(TrainRowsKernel, dim3(blocks), dim3(64 * kTrainWaves), 0, s, x, t,
+                       valid, batch, m->Pb, m->WT, m->P, m->omap, m->acts);
+    int32_t rc = CheckLaunch("TrainRowsKernel");
     if (rc != HWPA_OK) return rc;
-    hipLaunchKernelGGL(LossKernel, dim3((batch + 255) / 256), dim3(256), 0, s, m->Y, t, valid, batch, m->omap, m->dY,
-                       m->dYb, m->lossPer);
-    if ((rc = CheckLaunch("LossKernel")) != HWPA_OK) return rc;
-    hipLaunchKernelGGL(MeanKernel, dim3(1), dim3(256), 0, s, m->lossPer, batch, m->lossDev);
-    if ((rc = CheckLaunch("MeanKernel")) != HWPA_OK) return rc;
-    const uint16_t* Wb = m->Pb;
-    const int B = (int)batch;
-    // dW3[o][h] = sum_b dY[b][o] H2[b][h]
-    GemmArgs g = MakeGemm(MO, MH, B, m->dYb, 1, MO, m->H2, MH, 1);
-    if ((rc = GemmSplitK<false, false>(g, m->kPart, m->G + OFF_W3, s)) != HWPA_OK) return rc;
-    if ((rc = ColSum(m->dY, false, batch, MO, m->colPart, m->G + OFF_B3, s)) != HWPA_OK) return rc;
-    // dH2[b][h] = (sum_o dY[b][o] W3[o][h]) * [H2 > 0]
-    g = MakeGemm(B, MH, MO, m->dYb, MO, 1, Wb + OFF_W3, MH, 1);
-    g.mask = m->H2;
-    g.mk_m = MH;
-    g.mk_n = 1;
-    g.Cb = m->dH2;
-    g.c_m = MH;
-    g.c_n = 1;
-    if ((rc = Gemm<false, false, EPI_MASK_BF16>(g, s)) != HWPA_OK) return rc;
-    // dW2[o][i] = sum_b dH2[b][o] H1[b][i]
-    g = MakeGemm(MH, MH, B, m->dH2, 1, MH, m->H1, MH, 1);
-    if ((rc = GemmSplitK<false, false>(g, m->kPart, m->G + OFF_W2, s)) != HWPA_OK) return rc;
-    if ((rc = ColSum(m->dH2, true, batch, MH, m->colPart, m->G + OFF_B2, s)) != HWPA_OK) return rc;
-    // dH1[b][i] = (sum_o dH2[b][o] W2[o][i]) * [H1 > 0]
-    g = MakeGemm(B, MH, MH, m->dH2, MH, 1, Wb + OFF_W2, MH, 1);
-    g.mask = m->H1;
-    g.mk_m = MH;
-    g.mk_n = 1;
-    g.Cb = m->dH1;
-    g.c_m = MH;
-    g.c_n = 1;
-    if ((rc = Gemm<true, false, EPI_MASK_BF16>(g, s)) != HWPA_OK) return rc;
-    // dW1[o][i] = sum_b dH1[b][o] X[b][i]
-    g = MakeGemm(MH, MI, B, m->dH1, 1, MH, x, MI, 1);
-    if ((rc = GemmSplitK<false, false>(g, m->kPart, m->G + OFF_W1, s)) != HWPA_OK) return rc;
-    return ColSum(m->dH1, true, batch, MH, m->colPart, m->G + OFF_B1, s);
+    const dim3 grid(kGradTiles + 1), threads(64 * kGradWaves);
+    if (step)
+        hipLaunchKernelGGL(TrainGradKernel<true>, grid, threads, 0, s, m->acts, batch, nullptr, m->lossDev, *step);
+    else
+        hipLaunchKernelGGL(TrainGradKernel<false>, grid, threads, 0, s, m->acts, batch, m->G, m->lossDev, AdamArgs{});
+    return CheckLaunch("TrainGradKernel");
 }
 
 // Deterministic He-uniform initialisation from a 64-bit seed (biases zero).
@@ -836,12 +871,6 @@ int32_t MlpTargets(const hwpa_lane_hist* hist, const float* diag, uint32_t lanes
     return CheckLaunch("TargetsKernel");
 }
 
-int32_t MlpForward(const hwpa_initializer* m, const uint16_t* x, uint32_t rows, float* y, uint16_t* h1, uint16_t* h2,
-                   hipStream_t s)
-{
-    return Forward(m, x, rows, y, h1, h2, s);
-}
-
 int32_t MlpForwardFromHist(const hwpa_initializer* m, const hwpa_lane_hist* hist, uint32_t lanes, float* y,
                            hipStream_t s)
 {
@@ -865,7 +894,7 @@ int32_t hwpa_initializer_create(uint64_t seed, hwpa_initializer** out)
     if (rc == HWPA_OK) rc = DeviceAlloc((void**)&m->Ve, NPARAM * 4, "mlp moments");
     if (rc == HWPA_OK) rc = DeviceAlloc((void**)&m->lossDev, 16, "mlp loss");
     if (rc == HWPA_OK) rc = DeviceAlloc((void**)&m->omap, 20 * sizeof(float), "mlp output map");
-    if (rc == HWPA_OK) rc = DeviceAlloc((void**)&m->kPart, (size_t)kMaxSplit * MH * MH * 4, "mlp split-K partials");
+    if (rc == HWPA_OK) rc = DeviceAlloc((void**)&m->WT, NTRANS * 2, "mlp parameters");
     if (rc != HWPA_OK) {
         hwpa_initializer_destroy(m);
         return rc;
@@ -896,7 +925,6 @@ int32_t hwpa_initializer_destroy(hwpa_initializer* m)
 {
     if (!m) return HWPA_OK;
     (void)hipDeviceSynchronize();
-    FreeActs(m);
     FreeTrain(m);
     DeviceFree(m->P);
     DeviceFree(m->Pb);
@@ -905,7 +933,7 @@ int32_t hwpa_initializer_destroy(hwpa_initializer* m)
     DeviceFree(m->Ve);
     DeviceFree(m->lossDev);
     DeviceFree(m->omap);
-    DeviceFree(m->kPart);
+    DeviceFree(m->WT);
     LearnedWsFree(m->ws);
     delete m;
     return HWPA_OK;
@@ -930,7 +958,8 @@ int32_t hwpa_initializer_set_params(hwpa_initializer* m, const float* host_param
     HWPA_HIP(hipMemset(m->Ve, 0, NPARAM * 4));
     HWPA_HIP(hipMemset(m->G, 0, NPARAM * 4));
     m->step = 0;
-    hipLaunchKernelGGL(ToBf16Kernel, dim3((NPARAM + 255) / 256), dim3(256), 0, nullptr, m->P, m->Pb, (uint32_t)NPARAM);
+    hipLaunchKernelGGL(ToBf16Kernel, dim3((NPARAM + 255) / 256), dim3(256), 0, nullptr, m->P, m->Pb, m->WT,
+                       (uint32_t)NPARAM);
     int32_t rc = CheckLaunch("ToBf16Kernel");
     if (rc != HWPA_OK) return rc;
     HWPA_HIP(hipDeviceSynchronize());
@@ -985,8 +1014,7 @@ int32_t hwpa_mlp_forward(hwpa_initializer* m, const uint16_t* d_x, uint32_t rows
 {
     if (!m || !d_x || !d_y || rows == 0) return Fail(HWPA_ERR_INVALID_ARG, "mlp forward: null argument or no rows");
     if (((uintptr_t)d_x & 15) != 0) return Fail(HWPA_ERR_INVALID_ARG, "mlp forward: input must be 16-byte aligned");
-    // Inference keeps the hidden activations on chip (the fused kernel writes them only for training).
-    return Forward(m, d_x, rows, d_y, nullptr, nullptr, (hipStream_t)stream);
+    return Forward(m, d_x, rows, d_y, (hipStream_t)stream);
 }
 
 int32_t hwpa_mlp_forward_hist(hwpa_initializer* m, const hwpa_lane_hist* d_hist, uint32_t lanes, float* d_y,
@@ -1004,7 +1032,7 @@ int32_t hwpa_mlp_gradients(hwpa_initializer* m, const uint16_t* d_x, const float
     int32_t rc = EnsureBatch(m, batch);
     if (rc != HWPA_OK) return rc;
     hipStream_t s = (hipStream_t)stream;
-    if ((rc = Backward(m, d_x, d_t, d_valid, batch, s)) != HWPA_OK) return rc;
+    if ((rc = Backward(m, d_x, d_t, d_valid, batch, nullptr, s)) != HWPA_OK) return rc;
     if (d_grads) HWPA_HIP(hipMemcpyAsync(d_grads, m->G, NPARAM * 4, hipMemcpyDeviceToDevice, s));
     if (d_loss) HWPA_HIP(hipMemcpyAsync(d_loss, m->lossDev, 4, hipMemcpyDeviceToDevice, s));
     return HWPA_OK;
@@ -1019,14 +1047,13 @@ int32_t hwpa_mlp_train_step(hwpa_initializer* m, const uint16_t* d_x, const floa
     int32_t rc = EnsureBatch(m, batch);
     if (rc != HWPA_OK) return rc;
     hipStream_t s = (hipStream_t)stream;
-    if ((rc = Backward(m, d_x, d_t, d_valid, batch, s)) != HWPA_OK) return rc;
-    m->step += 1;
+    const int64_t step = m->step + 1;
     const double b1 = 0.9, b2 = 0.999;
-    const float c1 = (float)(1.0 - std::pow(b1, (double)m->step));
-    const float c2 = (float)(1.0 - std::pow(b2, (double)m->step));
-    hipLaunchKernelGGL(AdamKernel, dim3((NPARAM + 255) / 256), dim3(256), 0, s, m->P, m->G, m->Mo, m->Ve, m->Pb,
-                       (uint32_t)NPARAM, lr, (float)b1, (float)b2, c1, c2, 1e-8f);
-    if ((rc = CheckLaunch("AdamKernel")) != HWPA_OK) return rc;
+    const float c1 = (float)(1.0 - std::pow(b1, (double)step));
+    const float c2 = (float)(1.0 - std::pow(b2, (double)step));
+    const AdamArgs adam{m->P, m->Mo, m->Ve, m->Pb, m->WT, lr, (float)b1, (float)b2, c1, c2, 1e-8f};
+    if ((rc = Backward(m, d_x, d_t, d_valid, batch, &adam, s)) != HWPA_OK) return rc;
+    m->step = step;
     if (d_loss) HWPA_HIP(hipMemcpyAsync(d_loss, m->lossDev, 4, hipMemcpyDeviceToDevice, s));
     return HWPA_OK;
 }

@@ -137,6 +137,41 @@ def test_gradients_match_oracle(H, gpu, batch):
         o += n
 
 
+@pytest.mark.parametrize("batch", [1, 31, 33, 2049, 32 * 256 + 1])
+def test_gradients_and_step_at_block_edges(H, gpu, batch):
+    """Batches around the 32-row blocks, the waves' shares of them and one block per workgroup: the
+    gradients, and one Adam step from zero moments, which is lr * g / (|g| + eps), and the loss, after
+    the step too (the transposed weights follow the parameters)."""
+    rng = np.random.default_rng(batch)
+    init = H.Initializer(seed=5)
+    p = init.params()
+    x, t = _realistic_batch(rng, batch)
+    valid = t[:, 11].astype(np.uint8)
+    d_x, d_t, d_v = _upload_bf16(H, x), H.dev_from_numpy(t), H.dev_from_numpy(valid)
+    d_g, d_l = H.dev_bytes(M.NPARAM * 4), H.dev_bytes(4)
+    for _ in range(2):
+        init.gradients(d_x, d_t, batch, d_g, d_l, d_valid=d_v)
+        H.sync()
+        g = H.to_numpy(d_g, np.float32, (M.NPARAM,))
+        loss = H.to_numpy(d_l, np.float32, (1,))[0]
+        L_ref, g_ref = M.gradients(p, x, t, valid=valid)
+        assert abs(loss - L_ref) <= 1e-4 * abs(L_ref)
+        o = 0
+        for name, shape in M.SIZES:
+            n = int(np.prod(shape))
+            a, b = g[o:o + n], g_ref[o:o + n]
+            assert np.linalg.norm(a - b) < 2e-2 * max(np.linalg.norm(b), 1e-30), name
+            o += n
+        if _ == 0:
+            init.train_step(d_x, d_t, batch, 1e-3, d_loss=d_l, d_valid=d_v)
+            H.sync()
+            assert H.to_numpy(d_l, np.float32, (1,))[0] == loss
+            q = init.params()
+            want = p - 1e-3 * g / (np.abs(g) + 1e-8)
+            assert np.max(np.abs(q - want)) < 2e-6
+            p = q
+
+
 def test_training_lowers_loss(H, gpu):
     """Adam on the GPU fits a teacher network's outputs."""
     rng = np.random.default_rng(4)
