@@ -309,6 +309,7 @@ struct EmExtra {
     float* diag;              // optional raw estimate [lane][HWPA_EM_DIAG_ROWS][64]
     const uint32_t* active;   // optional: number of valid ZMWs; lanes at or beyond it exit, and the
                               // last lane's missing ZMWs run as copies of its first one
+    uint32_t activeMin, activeMax;   // with active: the launch does nothing unless activeMin <= *active <= activeMax
     const uint8_t* laneSel;   // optional: only lanes whose 64 flags here are all set run
     float acceptConf;         // EM_LEARNED: minimum confidence to accept the capped EM
     float convTol;            // EM_LEARNED: relative log-likelihood convergence tolerance
@@ -381,6 +382,7 @@ __global__ __launch_bounds__(QUAD ? 4 * LS : LS, MINW) void DmeEstimateKernel(co
     int zin = z;   // the ZMW whose inputs this thread reads
     if (x.active) {
         const uint32_t valid = *x.active;
+        if (valid < x.activeMin || valid > x.activeMax) return;
         if ((uint32_t)lane * LS >= valid) return;
         if ((uint32_t)lane * LS + (uint32_t)z >= valid) zin = 0;
     }
@@ -1429,9 +1431,20 @@ int32_t DmeEstimateLearned(const hwpa_config& cfg, hwpa_initializer* mlp, Learne
     EmExtra q{};
     q.laneSel = w.fallback;
     if ((rc = EmLaunch<EM_PLAIN>(waves, lanes, s, hist, stats, models, nullptr, d, evolve, q)) != HWPA_OK) return rc;
-    // How many of these waves have work is known on the device only; it is seldom all of them.
+    // How many of these lanes have work is known on the device only; it is seldom all of them.
+    // Up to kEmQuadLanes of them are estimated by four threads per ZMW, so past that size, unless
+    // other pools need the SIMDs, two launches go out of which one has work (the other's waves end
+    // at once, 5 us).  300 lanes, over half of their ZMWs rejected: 1.21 ms, one launch 1.78.
     EmExtra p{};
     p.active = w.total;
+    p.activeMax = UINT32_MAX;
+    if (lanes > kEmQuadLanes && sideBySide <= 3ull * lanes) {
+        p.activeMax = kEmQuadLanes * (uint32_t)LS;
+        rc = EmLaunch<EM_PLAIN>(1, kEmQuadLanes, s, w.cHist, w.cStats, w.cModels, w.cIters, d, evolve, p);
+        if (rc != HWPA_OK) return rc;
+        p.activeMin = p.activeMax + 1;
+        p.activeMax = UINT32_MAX;
+    }
     rc = EmLaunch<EM_PLAIN>(std::min(waves, 3), lanes, s, w.cHist, w.cStats, w.cModels, w.cIters, d, evolve, p);
     if (rc != HWPA_OK) return rc;
     hipLaunchKernelGGL(FallbackScatterKernel, dim3(lanes), dim3(LS), 0, s, w.total, w.map, w.cModels, models);

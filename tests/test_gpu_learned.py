@@ -155,3 +155,23 @@ def test_learned_estimate_bit_exact_with_oracle(H, O, T, trained):
     print("lanes falling back whole %d, in part %d" % ((per_lane == 64).sum(), ((per_lane > 0) & (per_lane < 64)).sum()))
     assert per_lane[5] == 64 and per_lane[29] == 64
     assert ((per_lane > 0) & (per_lane < 64)).any()
+
+
+@pytest.mark.parametrize("lanes", [256, 257, 700, 2400])
+def test_learned_estimate_same_at_all_sizes(H, O, T, trained, lanes):
+    """A ZMW's estimate does not depend on the pool's size, though the EM's form does: the 48 lanes
+    of a case repeated up to `lanes`, so that the compact lanes come on either side of the size
+    at which four threads estimate a ZMW, give the 48 lanes' models over and over."""
+    from test_gpu_parity import _dev, _em_case
+    L = 48
+    cfg, h, s, m = _em_case(H, O, T, L, F, seed=405, tg=dict(snr_lo=4.0, snr_hi=20.0))
+    cfg.learned_init = 1
+    mfi, efi = (512, 1024), (1024, 1536)
+    idx = np.arange(lanes) % L
+    d_one, d_all = _dev(H, m), _dev(H, m[idx].copy())
+    n_one = H.dme_estimate_learned(cfg, trained, _dev(H, h), _dev(H, s), d_one, mfi, efi, L)
+    n_all = H.dme_estimate_learned(cfg, trained, _dev(H, h[idx].copy()), _dev(H, s[idx].copy()), d_all, mfi, efi, lanes)
+    print("\nlearned start: %d of %d ZMWs fell back" % (n_all, lanes * 64))
+    assert n_one * (lanes // L) <= n_all <= n_one * (lanes // L + 1)
+    one = H.to_numpy(d_one, T.LANE_MODEL, (L,))
+    assert H.to_numpy(d_all, T.LANE_MODEL, (lanes,)).tobytes() == one[idx].tobytes()
