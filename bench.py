@@ -66,9 +66,9 @@ BASELINE_TRAFFIC_BYTES = {0: (1899107.5 * 2.0 + 3912546.4) * 1024, 1: (1826757.8
                           2: (1830723.6 * 2.0 + 3814150.6) * 1024, 3: (1867174.7 * 2.0 + 3935758.5) * 1024,
                           4: (1988898.2 * 2.0 + 4063900.4) * 1024, 5: (1854085.6 * 2.0 + 3806584.1) * 1024}
 # The histogram fast pass's, keyed by its autotuner variant (after the deferred reset, as the
-# analyzer runs it: the counters start from zero and are only written); variants 0-15 (one wave
-# per lane and the multi-wave forms) from an earlier run of the same commands.
-HIST_TRAFFIC_BYTES = {0: (1073590.5 * 2.0 + 1392903.8) * 1024, 1: (1074663.3 * 2.0 + 1940203.7) * 1024,
+# analyzer runs it: the counters start from zero and are only written); variants 1-15 (one wave
+# per lane and the multi-wave forms) from an earlier run of the same commands; 0 is 19's kernel.
+HIST_TRAFFIC_BYTES = {0: (1164363.9 * 2.0 + 1246209.0) * 1024, 1: (1074663.3 * 2.0 + 1940203.7) * 1024,
                       2: (1073285.7 * 2.0 + 1265043.3) * 1024, 3: (1073762.7 * 2.0 + 1392934.5) * 1024,
                       4: (1074528.2 * 2.0 + 1940203.7) * 1024, 5: (1073305.1 * 2.0 + 1265043.3) * 1024,
                       6: (1074254.5 * 2.0 + 1392934.5) * 1024, 7: (1076842.1 * 2.0 + 1940203.7) * 1024,
@@ -79,7 +79,7 @@ HIST_TRAFFIC_BYTES = {0: (1073590.5 * 2.0 + 1392903.8) * 1024, 1: (1074663.3 * 2
                       16: (1138660.5 * 2.0 + 1246208.2) * 1024, 17: (1164246.4 * 2.0 + 1246211.4) * 1024,
                       18: (1146681.8 * 2.0 + 1246216.1) * 1024, 19: (1164363.9 * 2.0 + 1246209.0) * 1024,
                       20: (1261457.9 * 2.0 + 1246210.8) * 1024, 21: (1100022.0 * 2.0 + 1246220.1) * 1024}
-HIST_KERNELS = [(0, "HistAddKernel"), (9, "HistAddWavesKernel"), (16, "HistAddFullKernel")]
+HIST_KERNELS = [(0, "HistAddFullKernel"), (1, "HistAddKernel"), (9, "HistAddWavesKernel"), (16, "HistAddFullKernel")]
 # VALU-bound stages: algorithmic VALU lane-operations per ZMW-frame (labeler: 61 add /
 # compare / select of the sparse recursion + 13 state scores + ROI; EM at one estimate per
 # 512-frame chunk: 20 iterations x (301 x 5 x (exp + 8) + 300 x 5 x 12) = 4e5 per ZMW per
@@ -88,7 +88,7 @@ HIST_KERNELS = [(0, "HistAddKernel"), (9, "HistAddWavesKernel"), (16, "HistAddFu
 # the SQ_INSTS_VALU counts of profiles/analyzer_kernels_32768lanes_f512_sq_counters.md.
 VALU_PEAK_LANE_OPS = 256 * 2.4e9 * 128
 VALU_ALG_OPS = {"labels": 400.0, "dme": 4.0e5 / 512}
-VALU_ISSUED_PER_LANE_FRAME = {"labels": 440.5, "dme": 849.0}
+VALU_ISSUED_PER_LANE_FRAME = {"labels": 440.5, "dme": 821.4}
 STAGES = ["baseline", "aggregate", "histogram", "dme", "labels", "pulses", "metrics"]
 
 
