@@ -244,10 +244,9 @@ static int32_t DmeAddBatch(hwpa_analyzer* a, int32_t first_frame)
     return HWPA_OK;
 }
 
-extern "C" {
-
-int32_t hwpa_analyzer_create(uint32_t pool_id, uint32_t lanes, uint32_t frames, const hwpa_config* cfg,
-                             hwpa_analyzer** out)
+// batchLanes: lanes of all pools of the batch the analyzer belongs to (0: none).
+static int32_t CreateAnalyzer(uint32_t pool_id, uint32_t lanes, uint32_t frames, const hwpa_config* cfg,
+                              uint64_t batchLanes, hwpa_analyzer** out)
 {
     if (!cfg || !out || lanes == 0) return Fail(HWPA_ERR_INVALID_ARG, "analyzer_create: bad argument");
     *out = nullptr;
@@ -263,7 +262,7 @@ int32_t hwpa_analyzer_create(uint32_t pool_id, uint32_t lanes, uint32_t frames, 
     a->poolId = pool_id;
     a->lanes = lanes;
     a->frames = frames;
-    a->sideBySide = (uint32_t)std::min<uint64_t>(3ull * lanes, UINT32_MAX);
+    a->sideBySide = (uint32_t)std::min<uint64_t>(batchLanes ? batchLanes : 3ull * lanes, UINT32_MAX);
     a->baselinerLatency = BaselinerStartupLatency(*cfg);
     const uint32_t cpe = (std::max(cfg->min_frames_for_estimate, 1u) + frames - 1) / frames;
     a->dmeDelay = (pool_id % cpe) * frames;
@@ -309,7 +308,8 @@ int32_t hwpa_analyzer_create(uint32_t pool_id, uint32_t lanes, uint32_t frames, 
             return rc;
         }
     }
-    if ((rc = BaselinerCreate(*cfg, lanes, &a->bl)) != HWPA_OK || (rc = LabelerCreate(*cfg, lanes, frames, &a->lab)) != HWPA_OK ||
+    if ((rc = BaselinerCreate(*cfg, lanes, &a->bl)) != HWPA_OK ||
+        (rc = LabelerCreate(*cfg, lanes, frames, &a->lab, batchLanes)) != HWPA_OK ||
         (rc = PulserCreate(*cfg, lanes, &a->pul)) != HWPA_OK || (rc = MetricsCreate(*cfg, lanes, &a->met)) != HWPA_OK) {
         FreeAnalyzer(a);
         return rc;
@@ -339,6 +339,14 @@ int32_t hwpa_analyzer_create(uint32_t pool_id, uint32_t lanes, uint32_t frames, 
     }
     *out = a;
     return HWPA_OK;
+}
+
+extern "C" {
+
+int32_t hwpa_analyzer_create(uint32_t pool_id, uint32_t lanes, uint32_t frames, const hwpa_config* cfg,
+                             hwpa_analyzer** out)
+{
+    return CreateAnalyzer(pool_id, lanes, frames, cfg, 0, out);
 }
 
 int32_t hwpa_analyzer_destroy(hwpa_analyzer* a)
@@ -746,20 +754,16 @@ int32_t hwpa_batch_create(uint32_t n_pools, const uint32_t* pool_ids, const uint
     *out = nullptr;
     hwpa_batch* b = new (std::nothrow) hwpa_batch();
     if (!b) return Fail(HWPA_ERR_OOM, "out of host memory");
+    uint64_t allLanes = 0;
+    for (uint32_t i = 0; i < n_pools; ++i) allLanes += lanes[i];
     for (uint32_t i = 0; i < n_pools; ++i) {
         hwpa_analyzer* a = nullptr;
-        const int32_t rc = hwpa_analyzer_create(pool_ids[i], lanes[i], frames[i], &cfgs[i], &a);
+        const int32_t rc = CreateAnalyzer(pool_ids[i], lanes[i], frames[i], &cfgs[i], allLanes, &a);
         if (rc != HWPA_OK) {
             FreeBatch(b);
             return rc;
         }
         b->pools.push_back(a);
-    }
-    uint64_t allLanes = 0;
-    for (auto* a : b->pools) allLanes += a->lanes;
-    for (auto* a : b->pools) {
-        LabelerShare(a->lab, allLanes);
-        a->sideBySide = (uint32_t)std::min<uint64_t>(allLanes, UINT32_MAX);
     }
     b->joins.assign(n_pools, nullptr);
     bool ok = hipStreamCreate(&b->master) == hipSuccess;

@@ -143,10 +143,10 @@ int32_t MetricsProcess(hwpa_metrics* m, const hwpa_pulse* pulses, const uint32_t
                        int32_t* produced, hipStream_t s);
 
 struct LabelerDev;
-int32_t LabelerCreate(const hwpa_config& cfg, uint32_t lanes, uint32_t max_frames, LabelerDev** out);
+// sideBySide: lanes that run side by side with this labeler's, its own included (0: its own).
+int32_t LabelerCreate(const hwpa_config& cfg, uint32_t lanes, uint32_t max_frames, LabelerDev** out,
+                      uint64_t sideBySide = 0);
 void LabelerDestroy(LabelerDev* l);
-// Tells a labeler how many lanes run side by side with its own (its own included).
-void LabelerShare(LabelerDev* l, uint64_t lanes);
 int32_t LabelerRun(LabelerDev* l, const int16_t* traces, uint32_t frames, const hwpa_lane_model* models,
                    int16_t* labels, int16_t* latent_out, float* score, hipStream_t s);
 

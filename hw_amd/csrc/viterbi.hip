@@ -41,7 +41,7 @@ struct LabelerDev {
     TransVals T;
     float roiUpper, roiLower;
     uint32_t lanes, maxFrames;
-    bool quad = false;       // the buffer holds LabelQuadKernel's words too
+    bool quad = false;       // labeled by LabelQuadKernel unless tuned; the buffer holds its words too
     LabLaneState* state = nullptr;
     uint32_t* tb = nullptr;  // [lane][maxFrames + 16 + NS][LS]: predecessor words, then the anchor row;
                              // or (quad) 64-bit words [lane][maxFrames + 16][LS]
@@ -1058,7 +1058,7 @@ static bool PackTransition(const hwpa_transition& T, TransVals& v)
     return true;
 }
 
-int32_t LabelerCreate(const hwpa_config& cfg, uint32_t lanes, uint32_t max_frames, LabelerDev** out)
+int32_t LabelerCreate(const hwpa_config& cfg, uint32_t lanes, uint32_t max_frames, LabelerDev** out, uint64_t sideBySide)
 {
     if (max_frames < (uint32_t)NL) return Fail(HWPA_ERR_INVALID_ARG, "labeler: max_frames must be >= 24");
     hwpa_transition T;
@@ -1073,7 +1073,7 @@ int32_t LabelerCreate(const hwpa_config& cfg, uint32_t lanes, uint32_t max_frame
     l->lanes = lanes;
     l->maxFrames = max_frames;
     int32_t rc = DeviceAlloc((void**)&l->state, sizeof(LabLaneState) * lanes, "labeler state");
-    l->quad = lanes <= kQuadLanes;
+    l->quad = std::max<uint64_t>(lanes, sideBySide) <= kQuadLanes;
     if (rc == HWPA_OK) {
         const size_t rows = max_frames + HWPA_VITERBI_LOOKBACK;
         const size_t words = l->quad ? std::max<size_t>(rows + NS, 2 * rows) : rows + NS;
@@ -1098,11 +1098,6 @@ void LabelerDestroy(LabelerDev* l)
     DeviceFree(l->state);
     DeviceFree(l->tb);
     delete l;
-}
-
-void LabelerShare(LabelerDev* l, uint64_t lanes)
-{
-    l->quad = l->quad && lanes <= kQuadLanes;
 }
 
 int32_t LabelerRun(LabelerDev* l, const int16_t* traces, uint32_t frames, const hwpa_lane_model* models,

@@ -1,3 +1,4 @@
+import ctypes
 import os
 import sys
 
@@ -44,3 +45,10 @@ def gen_traces(O, T, H, lanes, frames, chunks, seed=7, **kw):
     p = H.tracegen_default(seed=seed, **kw)
     st = np.zeros(lanes, dtype=T.TRACEGEN_STATE)
     return [O.tracegen(p, lanes, frames, c * frames, st, c == 0) for c in range(chunks)]
+
+
+def free_bytes(H):
+    """Free device memory (the HIP runtime that the library is linked against)."""
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    assert H.lib.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    return free.value

@@ -6,6 +6,8 @@ pool stagger), and the learned-start estimator inside the graph."""
 import numpy as np
 import pytest
 
+from conftest import free_bytes
+
 pytestmark = pytest.mark.gpu
 
 STEPS = 9
@@ -149,3 +151,21 @@ def test_batch_pools_match_oracle(H, O, T, gpu):
     # the bench-cadence pools estimate every chunk after start-up; the reference-cadence
     # pool (start-up 2 chunks + stagger 2 + 2 pre-accumulation + 8 estimation) from step 13
     assert all(n >= 10 for n in estimates[:3]) and estimates[3] >= 1, estimates
+
+
+def test_batch_traceback_words_by_the_form_that_runs(H, gpu):
+    """Four threads per ZMW label pools of up to 512 lanes and take twice the traceback words; pools
+    of one batch count together, and a batch past that size, which never runs that form, does not
+    hold its words."""
+    def held(n):
+        before = free_bytes(H)
+        b = H.Batch([(i, 300, 512, H.bench_config(512)) for i in range(n)])
+        took = before - free_bytes(H)
+        del b
+        return took
+
+    held(1)                                     # what the first batch of a process brings with it
+    one, two = held(1), held(2)
+    words = 300 * 528 * 64 * 4                  # a second word per frame, 40.6 MB a pool
+    print("one pool %.1f MB, two %.1f MB" % (one / 1e6, two / 1e6))
+    assert 1.5 * words < 2 * one - two < 2.5 * words
