@@ -916,13 +916,15 @@ int32_t hwpa_batch_autotune(hwpa_batch* b, int32_t repeats)
 {
     if (!b) return Fail(HWPA_ERR_INVALID_ARG, "null batch");
     HWPA_HIP(hipStreamSynchronize(b->master));
+    uint64_t allLanes = 0;
+    for (const auto* a : b->pools) allLanes += a->lanes;
     for (size_t i = 0; i < b->pools.size(); ++i) {
         const hwpa_analyzer* a = b->pools[i];
         bool seen = false;
         for (size_t j = 0; j < i && !seen; ++j)
             seen = b->pools[j]->lanes == a->lanes && b->pools[j]->frames == a->frames;
         if (seen) continue;
-        const int32_t rc = hwpa_autotune(&a->cfg, a->lanes, a->frames, repeats, nullptr, 0);
+        const int32_t rc = Autotune(&a->cfg, a->lanes, a->frames, repeats, allLanes, nullptr, 0);
         if (rc != HWPA_OK) return rc;
     }
     return HWPA_OK;

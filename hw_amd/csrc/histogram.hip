@@ -821,12 +821,12 @@ int32_t HistAddVariant(int32_t variant, hwpa_lane_hist* hist, void* edge, const 
     if (reinterpret_cast<uintptr_t>(hist) % 16 != 0)
         return Fail(HWPA_ERR_INVALID_ARG, "hist_add: histograms must be 16-byte aligned");
     EdgeLane* e = (EdgeLane*)edge;
-    switch (variant) {
     // The choice for shapes that were not tuned: the fastest form at every one measured, 16 to
     // 32,768 lanes x 128 to 1024 frames (one wave per lane with 160 bins, the earlier choice,
     // takes 124 against 15 us at 64 lanes x 512 frames, 311 against 91 at 4,096, 1131 against
     // 341 at 16,384).
-    case 0: return HistAddFullLaunch<8, 8, 2>(hist, e, traces, frames, models, lanes, s, wrap);
+    if (variant == 0) variant = kHistDefault;
+    switch (variant) {
     case 1: return HistAddLaunch<16, 128>(hist, e, traces, frames, models, lanes, s, wrap);
     case 2: return HistAddLaunch<16, 192>(hist, e, traces, frames, models, lanes, s, wrap);
     case 3: return HistAddLaunch<8, 160>(hist, e, traces, frames, models, lanes, s, wrap);

@@ -83,10 +83,15 @@ int32_t HistAddWrap(hwpa_lane_hist* hist, void* edge, const int16_t* traces, uin
                     const hwpa_lane_model* models, uint32_t lanes, hipStream_t s);
 
 // Kernel shape variants chosen per (lanes, frames) by the autotuner; every
-// variant computes the same bits.  Variant 0 is the choice by size, for shapes not tuned.
+// variant computes the same bits.  Variant 0 is the choice for shapes not tuned: one of the numbered
+// forms (of the baseline filter a form of its own), but for the labelers that LabelerDefault names.
 enum TuneKernel { kTuneHistogram = 0, kTuneBaseline = 1, kTuneLabel = 2, kTunePulse = 3, kTuneKernels = 4 };
+constexpr int32_t kHistDefault = 19, kPulseDefault = 4;
 int32_t TuneVariants(int kernel);
 int32_t TuneGet(int kernel, uint32_t lanes, uint32_t frames);
+// hwpa_autotune for a pool of a batch with batchLanes lanes in all (0: a pool of its own).
+int32_t Autotune(const hwpa_config* cfg, uint32_t lanes, uint32_t frames, int32_t repeats, uint64_t batchLanes,
+                 float* ms, int32_t ms_len);
 void TuneSet(int kernel, uint32_t lanes, uint32_t frames, int32_t variant);
 int32_t HistAddVariant(int32_t variant, hwpa_lane_hist* hist, void* edge, const int16_t* traces, uint32_t frames,
                        const hwpa_lane_model* models, uint32_t lanes, hipStream_t s, bool wrap = true);
@@ -147,6 +152,8 @@ struct LabelerDev;
 int32_t LabelerCreate(const hwpa_config& cfg, uint32_t lanes, uint32_t max_frames, LabelerDev** out,
                       uint64_t sideBySide = 0);
 void LabelerDestroy(LabelerDev* l);
+// The numbered variant an untuned labeler runs, 0 where that is LabelQuadKernel.
+int32_t LabelerDefault(const LabelerDev* l, uint32_t frames);
 int32_t LabelerRun(LabelerDev* l, const int16_t* traces, uint32_t frames, const hwpa_lane_model* models,
                    int16_t* labels, int16_t* latent_out, float* score, hipStream_t s);
 

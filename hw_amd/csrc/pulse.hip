@@ -296,7 +296,8 @@ int32_t PulserRun(PulserDev* p, const int16_t* labels, const int16_t* latent, co
     // every shape measured, 16 to 16,384 lanes x 128 to 1024 frames (records written at the frame
     // that ends them, 8 x 1, the earlier choice: 206 against 104 us at 64 lanes x 512 frames, 501
     // against 302 at 4,096, 1680 against 1154 at 16,384).
-    switch (TuneGet(kTunePulse, p->lanes, frames)) {
+    const int32_t tuned = TuneGet(kTunePulse, p->lanes, frames);
+    switch (tuned == 0 ? kPulseDefault : tuned) {
     case 1: HWPA_PULSE_LAUNCH(8, 2, false); break;
     case 2: HWPA_PULSE_LAUNCH(16, 2, false); break;
     case 3: HWPA_PULSE_LAUNCH(8, 1, true); break;
@@ -308,7 +309,7 @@ int32_t PulserRun(PulserDev* p, const int16_t* labels, const int16_t* latent, co
     case 10: HWPA_PULSE_LAUNCH(4, 12, true); break;
     case 11: HWPA_PULSE_LAUNCH(8, 4, true); break;
     case 12: HWPA_PULSE_LAUNCH(2, 16, true); break;
-    default: HWPA_PULSE_LAUNCH(8, 2, true); break;   // 0 and 4
+    default: HWPA_PULSE_LAUNCH(8, 2, true); break;   // kPulseDefault
     }
 #undef HWPA_PULSE_LAUNCH
     return CheckLaunch("PulseKernel");

@@ -121,6 +121,14 @@ int32_t hwpa_tune_get(int32_t kernel, uint32_t lanes, uint32_t frames, int32_t* 
 int32_t hwpa_autotune(const hwpa_config* cfg, uint32_t lanes, uint32_t frames, int32_t repeats, float* ms,
                       int32_t ms_len)
 {
+    return Autotune(cfg, lanes, frames, repeats, 0, ms, ms_len);
+}
+
+}  // extern "C"
+
+int32_t hwpa::Autotune(const hwpa_config* cfg, uint32_t lanes, uint32_t frames, int32_t repeats, uint64_t batchLanes,
+                       float* ms, int32_t ms_len)
+{
     if (!cfg || lanes == 0 || frames == 0 || repeats <= 0) return Fail(HWPA_ERR_INVALID_ARG, "autotune: bad argument");
     int32_t rc = hwpa_config_validate(cfg);
     if (rc != HWPA_OK) return rc;
@@ -160,7 +168,8 @@ int32_t hwpa_autotune(const hwpa_config* cfg, uint32_t lanes, uint32_t frames, i
     LabelerDev* lab = nullptr;
     PulserDev* pul = nullptr;
     if (stages) {
-        if ((rc = LabelerCreate(*cfg, lanes, frames, &lab)) != HWPA_OK) return rc;
+        // The labeler of such a pool, so that what is timed as its default is what it will run.
+        if ((rc = LabelerCreate(*cfg, lanes, frames, &lab, batchLanes)) != HWPA_OK) return rc;
         if ((rc = PulserCreate(*cfg, lanes, &pul)) != HWPA_OK) {
             LabelerDestroy(lab);
             return rc;
@@ -193,11 +202,26 @@ int32_t hwpa_autotune(const hwpa_config* cfg, uint32_t lanes, uint32_t frames, i
     }
 
     std::vector<float> times;
+    // Histogram inputs: this shape's baselined traces, bounds and models from its stats.
+    if ((rc = BaselinerRun(bl, raw, frames, bls, st, s)) != HWPA_OK) return rc;
+    if ((rc = DmeInitModels(*cfg, st, models, lanes, s)) != HWPA_OK) return rc;
+    if ((rc = EdgeStateInit(edge, lanes, s)) != HWPA_OK) return rc;
     for (int kernel = 0; kernel < kTuneKernels; ++kernel) {
         const int nv = TuneVariants(kernel);
+        // Variant 0 where it stands for a numbered form: that one is timed, and kept by its own
+        // number, so that the table means the same form to every pool.
+        int same = 0;
+        if (kernel == kTuneHistogram) same = kHistDefault;
+        else if (kernel == kTunePulse && stages) same = kPulseDefault;
+        else if (kernel == kTuneLabel && stages) same = LabelerDefault(lab, frames);
+        const size_t first = times.size();
         int best = 0;
         float bestMs = -1.0f;
         for (int v = 0; v < nv; ++v) {
+            if (v == 0 && same != 0) {
+                times.push_back(0.0f);   // of variant `same`, below
+                continue;
+            }
             float t = -1.0f;
             if (kernel == kTuneBaseline) {
                 TuneSet(kTuneBaseline, lanes, frames, v);
@@ -216,12 +240,6 @@ int32_t hwpa_autotune(const hwpa_config* cfg, uint32_t lanes, uint32_t frames, i
                     });
                 }
             } else {
-                // Histogram inputs: this shape's baselined traces, bounds and models from its stats.
-                if (v == 0) {
-                    if ((rc = BaselinerRun(bl, raw, frames, bls, st, s)) != HWPA_OK) return rc;
-                    if ((rc = DmeInitModels(*cfg, st, models, lanes, s)) != HWPA_OK) return rc;
-                    if ((rc = EdgeStateInit(edge, lanes, s)) != HWPA_OK) return rc;
-                }
                 // As the analyzer runs it after an estimate: the reset leaves the zero
                 // counters to the add.
                 t = TimeIt(s, repeats, [&]() {
@@ -236,6 +254,7 @@ int32_t hwpa_autotune(const hwpa_config* cfg, uint32_t lanes, uint32_t frames, i
                 best = v;
             }
         }
+        times[first] = times[first + same];
         TuneSet(kernel, lanes, frames, best);
     }
     if (ms) {
@@ -244,5 +263,3 @@ int32_t hwpa_autotune(const hwpa_config* cfg, uint32_t lanes, uint32_t frames, i
     HWPA_HIP(hipStreamSynchronize(s));
     return HWPA_OK;
 }
-
-}  // extern "C"

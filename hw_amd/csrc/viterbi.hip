@@ -1100,6 +1100,16 @@ void LabelerDestroy(LabelerDev* l)
     delete l;
 }
 
+// Four threads per ZMW for small pools (kQuadLanes), <16, 4> for 4,096 lanes and more of chunks up to
+// 512 frames (4,096 x 512: 1.17 ms; <8, 1> 1.19, and <16, 1>, the earlier default, 1.25), else <8, 1>
+// (1,024 x 512: 0.49 ms; <16, 4> 0.53, <16, 1> 0.50; 4,096 x 1024, where the ROI words in LDS limit
+// the waves per SIMD anyway: 2.95 ms; <16, 4> 3.41).
+int32_t LabelerDefault(const LabelerDev* l, uint32_t frames)
+{
+    if (l->quad) return 0;
+    return (l->lanes >= 4096 && frames <= 512) ? 3 : 1;
+}
+
 int32_t LabelerRun(LabelerDev* l, const int16_t* traces, uint32_t frames, const hwpa_lane_model* models,
                    int16_t* labels, int16_t* latent_out, float* score, hipStream_t s)
 {
@@ -1110,28 +1120,20 @@ int32_t LabelerRun(LabelerDev* l, const int16_t* traces, uint32_t frames, const 
     const int nroi = (int)frames + HWPA_VITERBI_LOOKBACK + HWPA_ROI_STITCH;
     const size_t lds = (size_t)((nroi + 15) / 16) * LS * sizeof(uint32_t);
     // Variants: frames per prefetched batch x registers held to 4 waves per SIMD; 0 is the choice
-    // by size: four threads per ZMW for small pools (above), <16, 4> for 4,096 lanes and more of
-    // chunks up to 512 frames (4,096 x 512: 1.17 ms; <8, 1> 1.19, and <16, 1>, the earlier
-    // default, 1.25), else <8, 1> (1,024 x 512: 0.49 ms; <16, 4> 0.53, <16, 1> 0.50; 4,096 x 1024,
-    // where the ROI words in LDS limit the waves per SIMD anyway: 2.95 ms; <16, 4> 3.41).
+    // by size.
 #define HWPA_LABEL_LAUNCH(PB, W)                                                                                   \
     hipLaunchKernelGGL((LabelKernel<PB, W>), dim3(l->lanes), dim3(LS), lds, s, traces, (int)frames, models,        \
                        l->state, l->tb, (int)(l->maxFrames + HWPA_VITERBI_LOOKBACK + NS), labels, latent_out,      \
                        score, l->T, l->roiUpper, l->roiLower)
-    switch (TuneGet(kTuneLabel, l->lanes, frames)) {
+    const int32_t tuned = TuneGet(kTuneLabel, l->lanes, frames);
+    switch (tuned == 0 ? LabelerDefault(l, frames) : tuned) {
     case 1: HWPA_LABEL_LAUNCH(8, 1); break;
     case 2: HWPA_LABEL_LAUNCH(8, 4); break;
     case 3: HWPA_LABEL_LAUNCH(16, 4); break;
     default:
-        if (l->quad)
-            hipLaunchKernelGGL(LabelQuadKernel, dim3(l->lanes), dim3(4 * LS), lds, s, traces, (int)frames, models,
-                               l->state, reinterpret_cast<uint16_t*>(l->tb),
-                               (int)(l->maxFrames + HWPA_VITERBI_LOOKBACK), labels, latent_out, score, l->T,
-                               l->roiUpper, l->roiLower);
-        else if (l->lanes >= 4096 && frames <= 512)
-            HWPA_LABEL_LAUNCH(16, 4);
-        else
-            HWPA_LABEL_LAUNCH(8, 1);
+        hipLaunchKernelGGL(LabelQuadKernel, dim3(l->lanes), dim3(4 * LS), lds, s, traces, (int)frames, models,
+                           l->state, reinterpret_cast<uint16_t*>(l->tb), (int)(l->maxFrames + HWPA_VITERBI_LOOKBACK),
+                           labels, latent_out, score, l->T, l->roiUpper, l->roiLower);
         break;
     }
 #undef HWPA_LABEL_LAUNCH

@@ -137,7 +137,8 @@ int32_t hwpa_batch_sync(hwpa_batch* b);
 /* [0] steps run, [1] graph instantiations, [2] in-place graph updates. */
 int32_t hwpa_batch_graph_stats(const hwpa_batch* b, uint64_t stats[3]);
 
-/* Autotunes every pool's shape (hwpa_autotune on its lanes, frames, config). */
+/* Autotunes every pool's shape (hwpa_autotune on its lanes, frames, config), timing the labeler as
+ * a pool of this batch runs it. */
 int32_t hwpa_batch_autotune(hwpa_batch* b, int32_t repeats);
 
 /* ---- kernel-shape autotuner (no reference counterpart) -------------------
@@ -152,10 +153,14 @@ int32_t hwpa_batch_autotune(hwpa_batch* b, int32_t repeats);
  * per batch x batches in the load ring x record queue: the default, then 8x2, 16x2 writing records
  * directly; 8x1, 8x2, 4x2, 4x1, 4x4, 8x3, 4x8, 4x12, 8x4, 2x16 writing them through an LDS queue).
  * The launchers look up the variant for their (lanes, frames);
- * unset shapes use variant 0, the library's choice by the shape's size.  hwpa_autotune times every variant on
+ * unset shapes use variant 0, the library's choice by the shape's size: histogram 19, pulses 4, labels 3 for
+ * 4,096 lanes and more of chunks up to 512 frames, else 1; pools of at most 512 lanes (those of one batch
+ * counted together) are labeled by a form of their own, four threads per ZMW, which has no other number.
+ * hwpa_autotune times every variant on
  * synthetic traces of the shape (`repeats` timed runs each, HIP events) and
- * keeps the fastest; ms (optional, ms_len entries) receives the mean times
- * of the variants of kernel 0, then 1, 2 and 3. */
+ * keeps the fastest, by its own number where 0 stands for one; ms (optional, ms_len entries) receives the
+ * mean times of the variants of kernel 0, then 1, 2 and 3.  It times the labeler of a pool on its
+ * own; for the pools of a batch use hwpa_batch_autotune. */
 int32_t hwpa_tune_variants(int32_t kernel, int32_t* count);
 int32_t hwpa_tune_set(int32_t kernel, uint32_t lanes, uint32_t frames, int32_t variant);
 int32_t hwpa_tune_get(int32_t kernel, uint32_t lanes, uint32_t frames, int32_t* variant);

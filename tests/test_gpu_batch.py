@@ -153,6 +153,24 @@ def test_batch_pools_match_oracle(H, O, T, gpu):
     assert all(n >= 10 for n in estimates[:3]) and estimates[3] >= 1, estimates
 
 
+def test_batch_autotune_keeps_forms_that_run(H, gpu):
+    """Variant 0 of the labeler is four threads per ZMW in a pool of 300 lanes, but not in a batch of
+    two such pools: the batch's tuner neither times nor keeps it there, and keeps the
+    histogram's and the pulses' default by its own number."""
+    frames = 160
+    b = H.Batch([(i, 300, frames, H.bench_config(frames)) for i in range(2)])
+    kernels = (H.TUNE_HISTOGRAM, H.TUNE_LABEL, H.TUNE_PULSE)
+    try:
+        b.autotune(1)
+        assert all(H.tune_get(k, 300, frames) > 0 for k in kernels)
+        ms = H.autotune(H.bench_config(frames), 300, frames, repeats=2)
+        assert ms["histogram"][0] == ms["histogram"][19] and ms["pulses"][0] == ms["pulses"][4]
+        assert ms["labels"][0] not in ms["labels"][1:]      # a pool on its own: a form of its own
+    finally:
+        for k in range(4):
+            H.tune_set(k, 300, frames, 0)
+
+
 def test_batch_traceback_words_by_the_form_that_runs(H, gpu):
     """Four threads per ZMW label pools of up to 512 lanes and take twice the traceback words; pools
     of one batch count together, and a batch past that size, which never runs that form, does not
