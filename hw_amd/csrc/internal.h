@@ -107,6 +107,7 @@ int32_t DmeEstimate(const hwpa_config& cfg, const hwpa_lane_hist* hist, const hw
 // for up to `lanes` lanes.
 struct LearnedWs {
     uint32_t lanes = 0;
+    int device = -1;                  // of a kept workspace (LearnedWsTake)
     float* y = nullptr;               // [Z][11] network output
     uint8_t* fallback = nullptr;      // [Z]
     uint32_t* cnt = nullptr;          // [lanes] fallback ZMWs per lane

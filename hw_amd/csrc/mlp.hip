@@ -537,20 +537,22 @@ struct hwpa_initializer {
 
 namespace hwpa {
 
-// An estimation's workspace: the one the initialiser keeps if it is large enough and not in use,
-// else a new one.  Allocating and freeing its ten buffers on every call took 0.4 ms of a
-// 4,096-lane estimation's 4.1.
+// An estimation's workspace: the one the initialiser keeps if it is large enough, on the current
+// device and not in use, else a new one.  Allocating and freeing its ten buffers on every call took
+// 0.4 ms of a 4,096-lane estimation's 4.1.  A kept one that does not serve is freed first, so a
+// call never needs more memory than its own workspace.
 int32_t LearnedWsTake(hwpa_initializer* m, uint32_t lanes, LearnedWs& w)
 {
+    int device = -1;
+    HWPA_HIP(hipGetDevice(&device));
     {
         std::lock_guard<std::mutex> g(m->wsMutex);
-        if (m->ws.lanes >= lanes) {
-            w = m->ws;
-            m->ws = LearnedWs{};
-            return HWPA_OK;
-        }
+        std::swap(w, m->ws);
     }
-    return LearnedWsAlloc(w, lanes);
+    if (w.lanes >= lanes && w.device == device) return HWPA_OK;
+    const int32_t rc = LearnedWsAlloc(w, lanes);   // (frees what w holds)
+    w.device = device;
+    return rc;
 }
 
 // Gives a workspace back once nothing uses it; the larger of it and the kept one stays (up to

@@ -355,7 +355,9 @@ int32_t hwpa_mlp_gradients(hwpa_initializer* m, const uint16_t* d_x, const float
 int32_t hwpa_mlp_train_step(hwpa_initializer* m, const uint16_t* d_x, const float* d_t, const uint8_t* d_valid,
                             uint32_t batch, float lr, float* d_loss, void* stream);
 /* Learned-start estimation of one pool: *fallback_count (host, optional)
- * receives the number of ZMWs re-estimated by the plain EM.  Synchronous. */
+ * receives the number of ZMWs re-estimated by the plain EM.  Synchronous.
+ * The initialiser keeps the call's workspace (50 KB a lane) for the next one, at most one and
+ * of at most 16,384 lanes, until it is destroyed or a call on it needs a larger one. */
 int32_t hwpa_dme_estimate_learned(const hwpa_config* cfg, hwpa_initializer* m, const hwpa_lane_hist* d_hist,
                                   const hwpa_baseliner_stats* d_stats, hwpa_lane_model* d_models,
                                   const int32_t model_fi[2], const int32_t est_fi[2], uint32_t lanes,

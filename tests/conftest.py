@@ -1,6 +1,7 @@
 import ctypes
 import os
 import sys
+import time
 
 import numpy as np
 import pytest
@@ -49,6 +50,8 @@ def gen_traces(O, T, H, lanes, frames, chunks, seed=7, **kw):
 
 def free_bytes(H):
     """Free device memory (the HIP runtime that the library is linked against)."""
+    H.sync()
+    time.sleep(0.3)      # the driver counts freed memory as free some milliseconds later
     free, total = ctypes.c_size_t(), ctypes.c_size_t()
     assert H.lib.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
     return free.value

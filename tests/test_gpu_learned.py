@@ -175,3 +175,30 @@ def test_learned_estimate_same_at_all_sizes(H, O, T, trained, lanes):
     assert n_one * (lanes // L) <= n_all <= n_one * (lanes // L + 1)
     one = H.to_numpy(d_one, T.LANE_MODEL, (L,))
     assert H.to_numpy(d_all, T.LANE_MODEL, (lanes,)).tobytes() == one[idx].tobytes()
+
+
+def test_learned_estimate_gives_a_small_workspace_back(H, O, T, gpu):
+    """The initialiser keeps a workspace between estimations; one that is too small is freed
+    before a larger one is allocated, and one of more than 16,384 lanes is not kept: after an
+    estimation of 2,048 lanes and one of 16,400, as much memory is free as before both."""
+    from conftest import free_bytes
+    from test_gpu_parity import _em_case
+    cfg, h, s, m = _em_case(H, O, T, 1, F, seed=406)
+    cfg.learned_init = 1
+    mfi, efi = (512, 1024), (1024, 1536)
+    net = H.Initializer(seed=2)
+    big = 16400
+    rep = lambda a: H.dev_from_numpy(np.broadcast_to(a, (big,)).copy())  # noqa: E731
+    d_h, d_s, d_m = rep(h), rep(s), rep(m)
+    warm = H.Initializer(seed=2)      # what the kernels of both sizes bring with their first launch
+    for n in (2048, big):
+        H.dme_estimate_learned(cfg, warm, d_h, d_s, d_m, mfi, efi, n)
+    del warm
+    before = free_bytes(H)
+    H.dme_estimate_learned(cfg, net, d_h, d_s, d_m, mfi, efi, 2048)
+    kept = before - free_bytes(H)
+    H.dme_estimate_learned(cfg, net, d_h, d_s, d_m, mfi, efi, big)
+    left = before - free_bytes(H)
+    print("kept %.1f MB after 2,048 lanes, %.1f MB after %d" % (kept / 1e6, left / 1e6, big))
+    assert kept > 2048 * T.LANE_HIST.itemsize
+    assert left < 8 << 20
