@@ -426,6 +426,8 @@ __global__ __launch_bounds__(QUAD ? 4 * LS : LS, MINW) void DmeEstimateKernel(co
     const float rpaMin = hw_minf(hw_minf(rpa[0], rpa[1]), hw_minf(rpa[2], rpa[3]));
 
     Model det = LoadModel(lm, zin);
+    // A missing ZMW reads the model of the lane's first, which another wave writes at its end.
+    if (QUAD && x.active) __syncthreads();
     det.conf *= evolve;
 
     // PrelimEstimate (DmeEmHost.cpp:161-214)
