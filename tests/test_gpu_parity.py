@@ -264,22 +264,37 @@ def _em_case(H, O, T, L, F, seed, cfg=None, tg=None):
     return cfg, hist.get(T.LANE_HIST), agg.get(T.BASELINER_STATS), models
 
 
-@pytest.mark.parametrize("seed", [1, 2])
-def test_dme_estimate_bit_exact(H, O, T, gpu, seed):
-    L, F = 4, 512
-    cfg, h, s, m = _em_case(H, O, T, L, F, seed)
+# Pool sizes of the EM's forms: four threads per ZMW, one thread with two and with three waves per SIMD.
+EM_FORMS = [4, 260, 2100]
+
+
+def _em_against_oracle(H, O, T, cfg, h, s, m, lanes, nan_equal=False):
+    """The lanes of a case repeated up to `lanes`, each against the oracle's estimate bit for bit
+    (nan_equal: one NaN is as good as another)."""
+    L = len(h)
     mfi, efi = (512, 1024), (1024, 1536)
     o_models, diag = O.dme_estimate(cfg, h, s, m, mfi, efi, want_diag=True, form="mirror")
-    d_models = _dev(H, m)
-    d_iters = H.dev_bytes(L * 4)
-    H.dme_estimate(cfg, _dev(H, h), _dev(H, s), d_models, mfi, efi, L, d_iters)
-    g_models = H.to_numpy(d_models, T.LANE_MODEL, (L,))
-    iters = H.to_numpy(d_iters, np.int32, (L,))
-    assert list(iters) == [diag[l].iterations_run for l in range(L)]
-    _eq_struct(g_models, o_models, "models")
+    at = np.arange(lanes) % L
+    d_models = _dev(H, m[at])
+    d_iters = H.dev_bytes(lanes * 4)
+    H.dme_estimate(cfg, _dev(H, h[at]), _dev(H, s[at]), d_models, mfi, efi, lanes, d_iters)
+    assert list(H.to_numpy(d_iters, np.int32, (lanes,))) == [diag[l].iterations_run for l in at]
+    g, o = H.to_numpy(d_models, T.LANE_MODEL, (lanes,)), o_models[at]
+    for f in (g, o) if nan_equal else ():
+        w = f.view(np.uint16)
+        w[(w & 0x7fff) > 0x7c00] = 0x7e00
+    _eq_struct(g, o, "models")
 
 
-def test_dme_estimate_recurrence_edge_paths_bit_exact(H, O, T, gpu):
+@pytest.mark.parametrize("lanes", EM_FORMS)
+@pytest.mark.parametrize("seed", [1, 2])
+def test_dme_estimate_bit_exact(H, O, T, gpu, seed, lanes):
+    cfg, h, s, m = _em_case(H, O, T, 4, 512, seed)
+    _em_against_oracle(H, O, T, cfg, h, s, m, lanes)
+
+
+@pytest.mark.parametrize("lanes", EM_FORMS)
+def test_dme_estimate_recurrence_edge_paths_bit_exact(H, O, T, gpu, lanes):
     """Histograms whose boundaries start far below every component (densities below
     FLT_MIN and rising at the first restarts of the E-step's density recurrence, so
     those blocks take exp at every boundary) and bins 8 or 16 times wider (ratios
@@ -292,22 +307,16 @@ def test_dme_estimate_recurrence_edge_paths_bit_exact(H, O, T, gpu):
     h["bin_size"][1, 1::4] *= 8.0
     h["bin_size"][2, 1::4] *= 16.0
     h["low_bound"][3, 1::4] -= 250.0 * bs[3, 1::4]
-    mfi, efi = (512, 1024), (1024, 1536)
-    o_models, diag = O.dme_estimate(cfg, h, s, m, mfi, efi, want_diag=True, form="mirror")
-    d_models = _dev(H, m)
-    d_iters = H.dev_bytes(L * 4)
-    H.dme_estimate(cfg, _dev(H, h), _dev(H, s), d_models, mfi, efi, L, d_iters)
-    iters = H.to_numpy(d_iters, np.int32, (L,))
-    assert list(iters) == [diag[l].iterations_run for l in range(L)]
-    _eq_struct(H.to_numpy(d_models, T.LANE_MODEL, (L,)), o_models, "models")
+    _em_against_oracle(H, O, T, cfg, h, s, m, lanes)
 
 
+@pytest.mark.parametrize("lanes", EM_FORMS)
 @pytest.mark.parametrize("shape", ["full_counters", "few_bins", "far_bounds", "nan_models"])
-def test_dme_estimate_block_paths_bit_exact(H, O, T, gpu, shape):
+def test_dme_estimate_block_paths_bit_exact(H, O, T, gpu, shape, lanes):
     """The E-step's block forms against the oracle: counters whose sum passes 2^24 (every bin
-    full), bins empty for a whole lane between occupied ones (branch per bin), and bins so wide
-    that the restarts' exponents leave the range of the unclamped exp, and ZMWs whose
-    start model is NaN (in which NaN equals NaN)."""
+    full), bins empty for a whole lane between occupied ones (with one thread per ZMW a branch per
+    bin), and bins so wide that the restarts' exponents leave the range of the unclamped exp, and
+    ZMWs whose start model is NaN (in which NaN equals NaN)."""
     L, F = 4, 512
     cfg, h, s, m = _em_case(H, O, T, L, F, 5)
     h, m = h.copy(), m.copy()
@@ -331,18 +340,7 @@ def test_dme_estimate_block_paths_bit_exact(H, O, T, gpu, shape):
     else:
         h["bin_size"][0:2, 5::16] *= np.float32(3e3)
         h["low_bound"][1, 7::16] = np.float32(-3e5)
-    mfi, efi = (512, 1024), (1024, 1536)
-    o_models, diag = O.dme_estimate(cfg, h, s, m, mfi, efi, want_diag=True, form="mirror")
-    d_models = _dev(H, m)
-    d_iters = H.dev_bytes(L * 4)
-    H.dme_estimate(cfg, _dev(H, h), _dev(H, s), d_models, mfi, efi, L, d_iters)
-    iters = H.to_numpy(d_iters, np.int32, (L,))
-    assert list(iters) == [diag[l].iterations_run for l in range(L)]
-    g_models = H.to_numpy(d_models, T.LANE_MODEL, (L,))
-    for f in (g_models, o_models):
-        w = f.view(np.uint16)
-        w[(w & 0x7fff) > 0x7c00] = 0x7e00
-    _eq_struct(g_models, o_models, "models")
+    _em_against_oracle(H, O, T, cfg, h, s, m, lanes, nan_equal=True)
 
 
 @pytest.mark.parametrize("lanes", [1, 256, 257, 2049, 3073, 4097])
@@ -361,19 +359,7 @@ def test_dme_estimate_forms_bit_exact(H, O, T, gpu, lanes, seed):
     h["bin_count"][2, 130:] = 0
     h["bin_size"][3, 5::16] *= np.float32(3e3)
     m["analogs"][:, 2]["means"][4, 9] = np.float16(np.nan).view(np.uint16)
-    mfi, efi = (512, 1024), (1024, 1536)
-    o_models, diag = O.dme_estimate(cfg, h, s, m, mfi, efi, want_diag=True, form="mirror")
-    at = np.arange(lanes) % L
-    d_models = _dev(H, m[at])
-    d_iters = H.dev_bytes(lanes * 4)
-    H.dme_estimate(cfg, _dev(H, h[at]), _dev(H, s[at]), d_models, mfi, efi, lanes, d_iters)
-    iters = H.to_numpy(d_iters, np.int32, (lanes,))
-    assert list(iters) == [diag[l].iterations_run for l in at]
-    g, o = H.to_numpy(d_models, T.LANE_MODEL, (lanes,)), o_models[at]
-    for f in (g, o):
-        w = f.view(np.uint16)
-        w[(w & 0x7fff) > 0x7c00] = 0x7e00
-    _eq_struct(g, o, "models")
+    _em_against_oracle(H, O, T, cfg, h, s, m, lanes, nan_equal=True)
 
 
 @pytest.fixture(params=[0, 1, 2, 3])
