@@ -172,6 +172,36 @@ def test_gradients_and_step_at_block_edges(H, gpu, batch):
             p = q
 
 
+@pytest.mark.parametrize("batch", [33, 2049, 2150, 32 * 256 + 1])
+def test_gradients_of_the_last_rows(H, gpu, batch):
+    """Batches whose gradient comes from their last rows alone, those that the last, partly filled pass
+    of TrainGradKernel's waves sums (2,048 rows a pass): without the confidence term only valid rows
+    count.  The gradients, and one Adam step taken from such a batch."""
+    rng = np.random.default_rng(batch)
+    init = H.Initializer(seed=5)
+    p = init.params()
+    omap = np.concatenate([np.zeros(6), np.ones(6), np.ones(7), [0.0]]).astype(np.float32)
+    init.set_output_map(omap[:6], omap[6:12], omap[12:])
+    x, t = _realistic_batch(rng, batch)
+    valid = (np.arange(batch) >= (batch - 1) // 2048 * 2048).astype(np.uint8)
+    d_x, d_t, d_v = _upload_bf16(H, x), H.dev_from_numpy(t), H.dev_from_numpy(valid)
+    d_g, d_l = H.dev_bytes(M.NPARAM * 4), H.dev_bytes(4)
+    init.gradients(d_x, d_t, batch, d_g, d_l, d_valid=d_v)
+    H.sync()
+    g = H.to_numpy(d_g, np.float32, (M.NPARAM,))
+    L_ref, g_ref = M.gradients(p, x, t, omap=omap, valid=valid)
+    assert abs(H.to_numpy(d_l, np.float32, (1,))[0] - L_ref) <= 1e-4 * abs(L_ref)
+    o = 0
+    for name, shape in M.SIZES:
+        n = int(np.prod(shape))
+        a, b = g[o:o + n], g_ref[o:o + n]
+        assert np.linalg.norm(b) > 0 and np.linalg.norm(a - b) < 2e-2 * np.linalg.norm(b), name
+        o += n
+    init.train_step(d_x, d_t, batch, 1e-3, d_loss=d_l, d_valid=d_v)
+    H.sync()
+    assert np.max(np.abs(init.params() - (p - 1e-3 * g / (np.abs(g) + 1e-8)))) < 2e-6
+
+
 def test_training_lowers_loss(H, gpu):
     """Adam on the GPU fits a teacher network's outputs."""
     rng = np.random.default_rng(4)
