@@ -160,24 +160,63 @@ def test_learned_estimate_bit_exact_with_oracle(H, O, T, trained, to_limit):
     assert per_lane[per_lane < 64].sum() % 64 != 0      # the last compact lane is partly filled
 
 
-@pytest.mark.parametrize("lanes", [256, 257, 700, 2400])
-def test_learned_estimate_same_at_all_sizes(H, O, T, trained, lanes):
+def _lanes_with(per_lane, partial, lanes):
+    """Lanes of a case, repeated, whose partly rejected ones hold `partial` rejected ZMWs in all, filled
+    up to `lanes` (None: as many as that takes) with lanes that are rejected whole."""
+    kinds = np.nonzero((per_lane > 0) & (per_lane < 64))[0]
+    out, left = [], partial
+    while left > 64 * 64:
+        out.append(kinds[len(out) % len(kinds)])
+        left -= per_lane[out[-1]]
+    last = {0: None}                       # sum -> the lane that reaches it
+    for total in range(1, left + 1):
+        for k in kinds:
+            if total - per_lane[k] in last:
+                last[total] = k
+                break
+    while left:
+        out.append(last[left])
+        left -= per_lane[out[-1]]
+    whole = np.nonzero(per_lane == 64)[0]
+    while lanes is not None and len(out) < lanes:
+        out.append(whole[len(out) % len(whole)])
+    return np.array(out)
+
+
+@pytest.mark.parametrize("lanes,partial", [(256, None), (257, None), (None, 16384), (None, 16385), (700, None),
+                                           (2400, None), (3100, 16384), (3100, 16385), (3100, None), (4096, None)])
+def test_learned_estimate_same_at_all_sizes(H, O, T, trained, lanes, partial):
     """A ZMW's estimate does not depend on the pool's size, though the EM's form does: the 48 lanes
-    of a case repeated up to `lanes`, so that the compact lanes come on either side of the size
-    at which four threads estimate a ZMW, give the 48 lanes' models over and over."""
+    of a case, some of them rejected whole, repeated up to `lanes`, or so that `partial` ZMWs are
+    compacted (four threads estimate a ZMW up to 256 compact lanes, 16,384 ZMWs), give the 48
+    lanes' models over and over.  3,073 to 4,096 lanes run four waves per SIMD."""
     from test_gpu_parity import _dev, _em_case
     L = 48
     cfg, h, s, m = _em_case(H, O, T, L, F, seed=405, tg=dict(snr_lo=4.0, snr_hi=20.0))
+    for l in (5, 29):                      # 100 frames per ZMW: insufficient data
+        h["bin_count"][l] = 0
+        h["bin_count"][l, 10] = 100
+        h["outlier_low"][l] = 0
+        h["outlier_high"][l] = 0
     cfg.learned_init = 1
     mfi, efi = (512, 1024), (1024, 1536)
-    idx = np.arange(lanes) % L
-    d_one, d_all = _dev(H, m), _dev(H, m[idx].copy())
-    n_one = H.dme_estimate_learned(cfg, trained, _dev(H, h), _dev(H, s), d_one, mfi, efi, L)
-    n_all = H.dme_estimate_learned(cfg, trained, _dev(H, h[idx].copy()), _dev(H, s[idx].copy()), d_all, mfi, efi, lanes)
-    print("\nlearned start: %d of %d ZMWs fell back" % (n_all, lanes * 64))
-    assert n_one * (lanes // L) <= n_all <= n_one * (lanes // L + 1)
-    one = H.to_numpy(d_one, T.LANE_MODEL, (L,))
-    assert H.to_numpy(d_all, T.LANE_MODEL, (lanes,)).tobytes() == one[idx].tobytes()
+    d_hist, d_y = _dev(H, h), H.dev_bytes(L * 64 * H.MLP_OUT * 4)
+    trained.forward_hist(d_hist, L, d_y)
+    y = H.to_numpy(d_y, np.float32, (L * 64, H.MLP_OUT))
+    one, fb, n_one = O.dme_estimate_learned(cfg, h, s, m, mfi, efi, y, trained.output_map())
+    per_lane = np.asarray(fb).reshape(L, 64).astype(np.int64).sum(axis=1)
+    idx = np.arange(lanes) % L if partial is None else _lanes_with(per_lane, partial, lanes)
+    compacted = per_lane[idx][per_lane[idx] < 64].sum()
+    print("\nlearned start: %d lanes, %d ZMWs compacted" % (len(idx), compacted))
+    if partial is None:
+        assert (compacted > 16384) == (len(idx) > 600)
+    else:
+        assert compacted == partial and len(idx) > 256
+    d_all = _dev(H, m[idx].copy())
+    n_all = H.dme_estimate_learned(cfg, trained, _dev(H, h[idx].copy()), _dev(H, s[idx].copy()), d_all, mfi, efi,
+                                   len(idx))
+    assert n_all == per_lane[idx].sum()
+    assert H.to_numpy(d_all, T.LANE_MODEL, (len(idx),)).tobytes() == one[idx].tobytes()
 
 
 def test_learned_estimate_gives_a_small_workspace_back(H, O, T, gpu):
