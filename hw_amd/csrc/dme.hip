@@ -1315,8 +1315,12 @@ constexpr uint32_t kEmQuadLanes = 256;
 // round suffices.  Pools that run side by side share the SIMDs (sideBySide, their lanes together):
 // there a launch with fewer waves per SIMD keeps others out, and 3 is the choice past 2,048 (six
 // pools of 365 to 2,048 lanes in one graph: 7.1 ms a step, 7.5 with each pool's own choice; three
-// pools of 2,000 lanes on their streams: 1.71 ms a chunk against 1.82).  Four threads per ZMW pay up
-// to three such pools of 256 lanes (200 lanes each: 0.53 ms a chunk against 0.56).
+// pools of 2,000 lanes on their streams: 1.71 ms a chunk against 1.82).  Analyzers always pass a count of
+// lanes, so 4 serves estimates without one.  Four threads per ZMW pay up to three pools of 256
+// lanes, which is what the hardware queues let run at a time (a chunk with them and with one thread,
+// us, for one, two, three, four, six and eight pools of 200 lanes: 1051, 625, 536, 659, 550, 585 and
+// 1425, 810, 563, 784, 566, 616; of 256 lanes: 1057, 783, 579, 706, 681, 670 and 1434, 825, 641, 838,
+// 644, 703).
 static int EmWavesPerSimd(uint32_t lanes, uint32_t sideBySide)
 {
     constexpr uint32_t kSimds = 1024;

@@ -51,8 +51,10 @@ struct LabelerDev {
 // issues 1.5 times the instructions of LabelKernel, in waves 2.6 times shorter, so it wins until
 // its waves fill the chip's issue slots (512 frames, quad against one thread per ZMW: 16 lanes
 // 0.20 against 0.50 ms, 512 lanes 0.32 against 0.52, 1,024 lanes 0.55 against 0.54, 4,096 lanes
-// 1.9 against 1.2; three pools of 300 lanes on their streams: 0.67 against 0.70 ms a chunk, of 600
-// lanes 0.87 against 0.84).  Pools of one batch count together (six pools of 365 to 2,048 lanes in
+// 1.9 against 1.2).  Pools on their own streams, us a chunk with quad and without, for one, three
+// and eight pools: 300 lanes 1565, 673, 724 and 1740, 703, 765; 400 lanes 1575, 736, 790 and 1755,
+// 728, 793; 512 lanes 1671, 805, 848 and 1846, 762, 828, which one pool gains more than
+// three lose.  Pools of one batch count together (six pools of 365 to 2,048 lanes in
 // one graph: 7.1 ms a step, 7.3 with the two smallest on four threads).
 constexpr uint32_t kQuadLanes = 512;
 
@@ -1101,9 +1103,12 @@ void LabelerDestroy(LabelerDev* l)
 }
 
 // Four threads per ZMW for small pools (kQuadLanes), <16, 4> for 4,096 lanes and more of chunks up to
-// 512 frames (4,096 x 512: 1.17 ms; <8, 1> 1.19, and <16, 1>, the earlier default, 1.25), else <8, 1>
-// (1,024 x 512: 0.49 ms; <16, 4> 0.53, <16, 1> 0.50; 4,096 x 1024, where the ROI words in LDS limit
-// the waves per SIMD anyway: 2.95 ms; <16, 4> 3.41).
+// 512 frames, else <8, 1>.  Four waves per SIMD pay once there are as many, 4,096 lanes (512 frames,
+// <8, 1> and <16, 4>: 1,024 lanes 0.49 and 0.53 ms, 2,048 0.66 and 0.68, 3,072 0.91 and 0.94, 4,096
+// 1.20 and 1.17, 8,192 2.23 and 2.18, 16,384 4.27 and 4.22; 256 frames: 3,072 0.50 and 0.51, 4,096
+// 0.66 and 0.64, 8,192 1.21 and 1.17), and as long as their ROI words fit a CU's LDS, up to 618 frames
+// (4,096 lanes: 576 frames 1.34 and 1.31, 640 frames 1.47 and 1.78, 1024 frames 2.96 and 3.47; 8,192
+// lanes: 576 frames 2.48 and 2.47, 640 frames 2.74 and 3.12): the line lies at the usual length below.
 int32_t LabelerDefault(const LabelerDev* l, uint32_t frames)
 {
     if (l->quad) return 0;
