@@ -49,9 +49,13 @@ def gen_traces(O, T, H, lanes, frames, chunks, seed=7, **kw):
 
 
 def free_bytes(H):
-    """Free device memory (the HIP runtime that the library is linked against)."""
+    """Free device memory (the HIP runtime that the library is linked against).  The driver counts
+    freed memory as free some milliseconds later, so the figure has to stand for 0.4 s."""
     H.sync()
-    time.sleep(0.3)      # the driver counts freed memory as free some milliseconds later
     free, total = ctypes.c_size_t(), ctypes.c_size_t()
-    assert H.lib.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
-    return free.value
+    seen = []
+    while len(seen) < 40 and len(set(seen[-5:])) != 1 or len(seen) < 5:
+        assert H.lib.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+        seen.append(free.value)
+        time.sleep(0.1)
+    return seen[-1]
